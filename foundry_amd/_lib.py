@@ -91,6 +91,9 @@ class LlamaModel(ctypes.Structure):
     ]
 
 
+_I64x4 = ctypes.c_int64 * 4
+
+
 class View(ctypes.Structure):
     """fh_view: a strided view (src/metal/args.rs:22-29), in elements."""
     _fields_ = [("offset", ctypes.c_int64), ("ndim", ctypes.c_int32), ("dims", ctypes.c_int64 * 4),
@@ -98,11 +101,7 @@ class View(ctypes.Structure):
 
     @staticmethod
     def of(shape, strides, offset: int = 0) -> "View":
-        v = View()
-        v.offset, v.ndim = int(offset), len(shape)
-        for d, (n, st) in enumerate(zip(shape, strides)):
-            v.dims[d], v.strides[d] = int(n), int(st)
-        return v
+        return View(int(offset), len(shape), _I64x4(*map(int, shape)), _I64x4(*map(int, strides)))
 
 
 class HipError(RuntimeError):
@@ -228,4 +227,6 @@ def decode_attention_workspace_bytes(batch: int, n_heads: int, n_kv: int, head_d
 
 def call(name: str, *args) -> None:
     """Calls an fh_* function and raises HipError on a non-OK status."""
-    check(getattr(load(), name)(*args))
+    status = getattr(_lib or load(), name)(*args)
+    if status:
+        check(status)

@@ -9,6 +9,7 @@
 #include <map>
 #include <set>
 #include <string>
+#include <unordered_map>
 #include <utility>
 #include <vector>
 
@@ -45,6 +46,18 @@ constexpr uint64_t kPackAreaBytes = 8ull * 16384 * 2 + (16384 / 64) * 8 * 4 + 20
 constexpr uint64_t kPartialAreaBytes = 128ull << 20;
 // K splits of a prompt-length GEMM at most (their f32 partials share the area).
 constexpr uint32_t kMaxGemmSplits = 8;
+// Freed blocks a device keeps for its next allocations: at most this many
+// bytes and blocks in all, and none larger than kPoolBlockBytes.
+constexpr uint64_t kPoolBytes = 512ull << 20;
+constexpr uint64_t kPoolBlockBytes = 128ull << 20;
+constexpr size_t kPoolBlocks = 256;
+// A kept block serves a request it exceeds by at most this or 1/8 of it.
+constexpr uint64_t kPoolSlack = 64ull << 10;
+
+struct PoolBlock {
+    uintptr_t base;
+    size_t capacity;
+};
 }  // namespace fh
 
 struct fh_device {
@@ -56,6 +69,14 @@ struct fh_device {
     void *partial_area = nullptr;  // kPartialAreaBytes, likewise
     // base address -> size of every live allocation this device made
     std::map<uintptr_t, size_t> allocs;
+    // Freed blocks kept for reuse, oldest first, and their bytes. All work on
+    // a block is on the device's one stream, so whatever still uses it when
+    // it is freed runs before anything the next owner enqueues. capacity:
+    // bytes behind every block the device holds, live, retired or kept (a
+    // reused block may exceed the size asked for).
+    std::vector<fh::PoolBlock> pool;
+    uint64_t pool_bytes = 0;
+    std::unordered_map<uintptr_t, size_t> capacity;
     uint64_t live_bytes = 0;
     uint64_t peak_bytes = 0;
     uint64_t run_peak_bytes = 0;

@@ -291,10 +291,10 @@ class HipDevice:
     def _run_standard(self, op, inputs, shape, dtype, out) -> None:
         """The reference's own Ops through the strided entry points
         (MetalDevice::run, src/metal/mod.rs:639-695)."""
-        h, dst = self.handle, ctypes.c_void_p(out.ptr)
+        h, dst = self.handle, out.ptr
 
         def base(o):
-            return ctypes.c_void_p(o.storage.ptr)
+            return o.storage.ptr
 
         def view(o):
             return ctypes.byref(o.layout.view())

@@ -109,7 +109,12 @@ int fh_device_stream(fh_device *dev, void **stream);
  * zero_fill != 0 the memory is cleared before any later op on the stream
  * reads it (Device::zeros). */
 int fh_alloc(fh_device *dev, size_t nbytes, int zero_fill, void **out);
-/* Frees an allocation of this device after the work queued on it ends.
+/* Frees an allocation of this device. Work already queued on the device's
+ * stream may still use the memory; it is then kept for later fh_alloc calls
+ * of the device (at most 512 MiB, blocks of at most 128 MiB, the oldest given
+ * back first, all of them when the driver runs out) or given back to the
+ * driver once that work ends. Memory in use on a stream of the caller's own
+ * must not be freed before that use ends.
  * A live graph retains every allocation its captured ops touched, as a
  * Metal command buffer retains its buffers (src/metal/mod.rs:280-282): the
  * allocation is then no longer usable by ops but stays allocated until the
@@ -124,7 +129,8 @@ int fh_download(fh_device *dev, void *dst, const void *src, size_t nbytes);
 /* ---- memory and profile counters (src/nn/primitive.rs:75-83) ----
  * Bytes counted: every live allocation (including retired ones a graph still
  * holds) plus the device's own work areas (the 33 MB of GEMV/GEMM partial
- * sums and the batched GEMV's x image), allocated at creation. */
+ * sums and the batched GEMV's x image), allocated at creation; freed blocks
+ * kept for reuse (fh_free) are not counted. */
 int fh_max_memory_allocated(const fh_device *dev, fh_allocated_memory *out);
 int fh_reset_run_memory_peak(fh_device *dev);
 int fh_run_memory_peak(const fh_device *dev, fh_allocated_memory *out);

@@ -15,12 +15,14 @@ inputs with numpy restatements of the Metal kernels' arithmetic:
 - matmul: within 1e-5 (F32) or one bf16 ulp plus 1e-5 (BF16) of float64,
   relative to max|out|.
 """
+import ctypes
 import math
 
 import numpy as np
 import pytest
 
 from foundry_amd import _lib
+from foundry_amd.device import HipDevice
 from foundry_amd.primitive import DType, TensorError
 from foundry_amd.tensor import Tensor
 from oracle import llama_ref as R
@@ -399,3 +401,50 @@ def test_strided_entry_points_reject_bad_views(device):
         _lib.call("fh_binary", device.handle, 0, int(DType.F32), ctypes.c_void_p(t.storage.ptr), ctypes.byref(ok),
                   ctypes.c_void_p(t.storage.ptr), ctypes.byref(other), ctypes.c_void_p(out.ptr))
     assert e.value.kind == "InvalidArgument"
+
+
+# block sizes around the allocator's rules: one byte, a size and one that
+# differs by the 64 KiB slack a kept block may exceed a request by (and one
+# byte more), and the largest block that is kept (128 MiB, and one byte more)
+@pytest.mark.parametrize("nbytes", [1, 255, 4096, (64 << 10) + 1, 3 << 20, 128 << 20, (128 << 20) + 1])
+def test_freed_blocks_are_reused_in_stream_order(nbytes):
+    """fh_free keeps blocks for later fh_alloc calls. Whatever the block held
+    or still serves on the stream: the old pointer is foreign at once, a
+    zeroed allocation reads as zeros, a request of another size is bounded by
+    its own size, queued work on the old owner's data is not disturbed, and
+    only live bytes are counted."""
+    dev = HipDevice(0)
+    try:
+        dev.synchronize()
+        base = dev.max_memory_allocated()["bytes"]
+        for size in (nbytes, max(1, nbytes - 100), nbytes + (64 << 10), nbytes + (64 << 10) + 1):
+            keep = dev.empty(nbytes)
+            src = dev.storage_from_bytes(np.full(nbytes, 0xA5, np.uint8).tobytes())
+            view = _lib.View.of((nbytes // 4,), (1,))
+            # keep = src on the stream, then src is freed before that copy has run
+            if nbytes >= 4:
+                _lib.call("fh_copy_strided", dev.handle, int(DType.U32), src.ptr, ctypes.byref(view), keep.ptr)
+            old = src.ptr
+            del src
+            if nbytes >= 4:
+                with pytest.raises(_lib.HipError) as e:
+                    _lib.call("fh_copy_strided", dev.handle, int(DType.U32), old, ctypes.byref(view), keep.ptr)
+                assert e.value.kind == "ForeignStorage"
+            new = dev.zeros(size)
+            host = np.full(size, 1, np.uint8)
+            _lib.call("fh_download", dev.handle, host.ctypes.data_as(ctypes.c_void_p), new.ptr, size)
+            assert not host.any()
+            with pytest.raises(_lib.HipError) as e:
+                _lib.call("fh_download", dev.handle, host.ctypes.data_as(ctypes.c_void_p), new.ptr, size + 1)
+            assert e.value.kind == "OutOfBounds"
+            got = np.zeros(nbytes // 4 * 4, np.uint8)
+            if nbytes >= 4:
+                _lib.call("fh_download", dev.handle, got.ctypes.data_as(ctypes.c_void_p), keep.ptr, got.nbytes)
+                assert (got == 0xA5).all()
+            dev.reset_run_memory_peak()
+            assert dev.run_memory_peak()["bytes"] == base + nbytes + size
+            del keep, new
+        dev.reset_run_memory_peak()
+        assert dev.run_memory_peak()["bytes"] == base
+    finally:
+        dev.close()
