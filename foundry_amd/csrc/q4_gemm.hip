@@ -26,6 +26,7 @@
 //   on every load's address.)
 #include "device.hpp"
 #include "q4_common.hpp"
+#include "q4_gemm.hpp"
 
 namespace fh {
 
@@ -290,48 +291,78 @@ __global__ __launch_bounds__(256) void gemm_split_reduce_kernel(const float *__r
     }
 }
 
-// 256 x 256 tiles, or 256 x 128 when the larger tile leaves CUs idle: each
-// weight element is still dequantised once per 256 rows of X, and the
-// down-projection shape (2048 x 3072 x 8192) gets 192 blocks instead of 96
-// (249 -> 186 us; the 2048 x 8192 x 3072 shape stays at 256 x 256, 139 us
-// against 164). When even the small tiles leave more than half the CUs idle
-// (prompt-length m such as 512 against n = 3072 or 5120), K is split over
-// up to kMaxGemmSplits ranges so that tiles x splits about fills the chip;
-// the splits' f32 partials go to `area` (kPartialAreaBytes) and
-// gemm_split_reduce_kernel adds them in order. launch_q4_gemm_deferred stops
-// before that add and returns the split count (1: y was written), so that a
-// consumer of y can add the partials itself, in the same order.
-uint32_t launch_q4_gemm_direct(hipStream_t stream, uint32_t cus, const uint16_t *x, uint32_t x_ld,
-                               const uint32_t *wq, const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t n,
-                               uint32_t k, void *y, int y_is_f32, void *area);
-
-uint32_t launch_q4_gemm_deferred(hipStream_t stream, uint32_t cus, const uint16_t *x, uint32_t x_ld,
-                                 const uint32_t *wq, const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t n,
-                                 uint32_t k, void *y, int y_is_f32, void *area) {
-    const uint64_t big = static_cast<uint64_t>((n + 255) / 256) * ((m + 255) / 256);
-    // 256 x 256 tiles fill the chip, or 3/4 of it over two K ranges: weights
-    // straight to the matrix cores (q4_gemm_direct.hip)
-    if (const uint32_t d = launch_q4_gemm_direct(stream, cus, x, x_ld, wq, s, b, m, n, k, y, y_is_f32, area)) return d;
-    if (big >= cus) {
-        launch_gemm_tile<256, 256, 2, 4>(stream, x, x_ld, wq, s, b, m, n, k, y, y_is_f32, 1);
-        return 1;
-    }
+// Tiles of q4_gemm_kernel: 256 x 256, or 256 x 128 when the larger tile leaves
+// CUs idle (each weight element is still dequantised once per 256 rows of X).
+// When even the small tiles leave more than half the CUs idle, K is split
+// over up to kMaxGemmSplits ranges of at least 4 steps so that tiles x splits
+// about fills the chip.
+static uint32_t staged_gemm_splits(uint32_t cus, uint32_t m, uint32_t n, uint32_t k, bool area) {
     const uint64_t tiles = static_cast<uint64_t>((n + 127) / 128) * ((m + 255) / 256);
     const uint64_t steps = k / kBK;
     uint64_t splits = 1;
-    if (area != nullptr && 2 * tiles <= cus) {
+    if (area && 2 * tiles <= cus) {
         splits = cus / tiles;
         if (splits > kMaxGemmSplits) splits = kMaxGemmSplits;
         if (splits > steps / 4) splits = steps / 4;  // at least 4 K steps per split
         while (splits > 1 && splits * m * n * 4 > kPartialAreaBytes) --splits;
         if (splits < 1) splits = 1;
     }
+    return static_cast<uint32_t>(splits);
+}
+
+// Estimated us of the 256-row kernels for a shape. The direct one takes about
+// 30 ns per value of K and round of 256 x 256 tiles (93 us at 2048 x 8192 x
+// 3072), the staged one 16 ns plus up to 9.5 ns more as its 256 x 128 tiles
+// fill the chip (512 x 5120 x 3072 over 3 ranges 37.7 us, 1024 x 5120 x 3072
+// in one 66.2 us); a K split adds the pass over its f32 partials.
+static double tiled_gemm_us(uint32_t cus, uint32_t x_ld, uint32_t m, uint32_t n, uint32_t k, bool area) {
+    const uint64_t big = static_cast<uint64_t>((n + 255) / 256) * ((m + 255) / 256);
+    const uint64_t small = static_cast<uint64_t>((n + 127) / 128) * ((m + 255) / 256);
+    const uint32_t direct = direct_gemm_splits(cus, x_ld, m, n, k, area);
+    const uint32_t splits = direct ? direct : big >= cus ? 1 : staged_gemm_splits(cus, m, n, k, area);
+    const uint64_t blocks = (direct || big >= cus ? big : small) * splits;
+    const double rounds = static_cast<double>((blocks + cus - 1) / cus);
+    const double fill = static_cast<double>(blocks) / (rounds * cus);
+    const double add = splits > 1 ? 3.0 + static_cast<double>(m) * n * 4 * splits / 6e6 : 0.0;
+    return 4.0 + rounds * k / splits * (direct ? 0.030 : 0.016 + 0.0095 * fill) + add;
+}
+
+// Which kernel a shape takes:
+// - few rows (q4_gemm_rows.hip) where its estimate is below the 256-row
+//   kernels' by 3% (both models above and there; measured, rows kernel
+//   against 256-row kernels: 32 x 28672 x 4096 27.2 against 75.8 us, 48 x 4096
+//   x 4096 8.8 / 20.5, 128 x 5120 x 3072 13.2 / 25.7, 256 x 3072 x 8192 24.1 /
+//   35.4, 512 x 3072 x 3072 21.8 / 29.5, 1024 x 3072 x 8192 88.2 / 101.5; on
+//   the other side of the line 1024 x 5120 x 3072 70.1 / 66.2, 256 x 16384 x
+//   3072 57.1 / 51.1);
+// - weights straight to the matrix cores (q4_gemm_direct.hip) where its
+//   256 x 256 tiles fill the chip, or 3/4 of it over two K ranges;
+// - q4_gemm_kernel otherwise.
+// launch_q4_gemm_deferred leaves a K split's f32 partials in `area`
+// (kPartialAreaBytes) and returns the split count (1: y was written), so that
+// a consumer of y can add the partials itself, in the order
+// gemm_split_reduce_kernel adds them.
+uint32_t launch_q4_gemm_deferred(hipStream_t stream, uint32_t cus, const uint16_t *x, uint32_t x_ld,
+                                 const uint32_t *wq, const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t n,
+                                 uint32_t k, void *y, int y_is_f32, void *area) {
+    const RowsPlan rows = plan_q4_gemm_rows(cus, x_ld, s, b, m, n, k);
+    if (rows.ct != 0 && 1.03 * rows.us < tiled_gemm_us(cus, x_ld, m, n, k, area != nullptr)) {
+        launch_q4_gemm_rows(stream, rows, x, x_ld, wq, s, b, m, n, k, y, y_is_f32);
+        return 1;
+    }
+    if (const uint32_t d = launch_q4_gemm_direct(stream, cus, x, x_ld, wq, s, b, m, n, k, y, y_is_f32, area)) return d;
+    const uint64_t big = static_cast<uint64_t>((n + 255) / 256) * ((m + 255) / 256);
+    if (big >= cus) {
+        launch_gemm_tile<256, 256, 2, 4>(stream, x, x_ld, wq, s, b, m, n, k, y, y_is_f32, 1);
+        return 1;
+    }
+    const uint32_t splits = staged_gemm_splits(cus, m, n, k, area != nullptr);
     if (splits == 1) {
         launch_gemm_tile<256, 128, 4, 2>(stream, x, x_ld, wq, s, b, m, n, k, y, y_is_f32, 1);
         return 1;
     }
-    launch_gemm_tile<256, 128, 4, 2>(stream, x, x_ld, wq, s, b, m, n, k, area, 1, static_cast<uint32_t>(splits));
-    return static_cast<uint32_t>(splits);
+    launch_gemm_tile<256, 128, 4, 2>(stream, x, x_ld, wq, s, b, m, n, k, area, 1, splits);
+    return splits;
 }
 
 void launch_q4_gemm(hipStream_t stream, uint32_t cus, const uint16_t *x, uint32_t x_ld, const uint32_t *wq,

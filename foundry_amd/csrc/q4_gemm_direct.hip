@@ -42,6 +42,7 @@
 #include "decoder_common.hpp"
 #include "device.hpp"
 #include "q4_common.hpp"
+#include "q4_gemm.hpp"
 
 namespace fh {
 
@@ -516,22 +517,17 @@ static void direct_lds_opt_in() {
     }
 }
 
-// Launches the direct-weight GEMM when it applies: 256 x 256 tiles that fill
-// the chip (the 2048 x 8192 x 3072 gate/up shape has exactly 256), or fill
-// at least 3/4 of it over two K ranges (the 2048 x 3072 x 8192 down shape:
-// 96 tiles, 192 blocks), k a multiple of 512 per range (whole scale/bias
-// chunks) and every per-lane byte offset within 32 bits. Returns 0 when it
-// does not apply, 1 when y was written, 2 when the two ranges' f32 partials
-// were left in `area` ([2][m][n], for the caller to add in order).
-uint32_t launch_q4_gemm_direct(hipStream_t stream, uint32_t cus, const uint16_t *x, uint32_t x_ld,
-                               const uint32_t *wq, const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t n,
-                               uint32_t k, void *y, int y_is_f32, void *area) {
-    const uint32_t tiles_m = (m + kDBM - 1) / kDBM, tiles_n = (n + kDBN - 1) / kDBN;
-    const uint64_t tiles = static_cast<uint64_t>(tiles_m) * tiles_n;
+// K ranges of the direct-weight GEMM where it applies: 256 x 256 tiles that
+// fill the chip (the 2048 x 8192 x 3072 gate/up shape has exactly 256; one
+// range), or fill at least 3/4 of it over two K ranges (the 2048 x 3072 x
+// 8192 down shape: 96 tiles, 192 blocks), k a multiple of 512 per range
+// (whole scale/bias chunks) and every per-lane byte offset within 32 bits.
+// 0 where it does not apply.
+uint32_t direct_gemm_splits(uint32_t cus, uint32_t x_ld, uint32_t m, uint32_t n, uint32_t k, bool area) {
+    const uint64_t tiles = static_cast<uint64_t>((m + kDBM - 1) / kDBM) * ((n + kDBN - 1) / kDBN);
     uint32_t splits = 1;
     if (tiles < cus) {
-        if (area == nullptr || 8 * tiles < 3ull * cus || k % (2 * kDSbGroups * kDBK) != 0 ||
-            2ull * m * n * 4 > kPartialAreaBytes)
+        if (!area || 8 * tiles < 3ull * cus || k % (2 * kDSbGroups * kDBK) != 0 || 2ull * m * n * 4 > kPartialAreaBytes)
             return 0;
         splits = 2;
     }
@@ -539,6 +535,19 @@ uint32_t launch_q4_gemm_direct(hipStream_t stream, uint32_t cus, const uint16_t 
     if (tiles > 0x7FFFFFFFull || k % (kDSbGroups * kDBK) != 0 || k == 0 || m == 0) return 0;
     if (static_cast<uint64_t>(m) * x_ld * 2 >= (1ull << 32) || static_cast<uint64_t>(n) * k / 2 >= (1ull << 32))
         return 0;
+    return splits;
+}
+
+// Launches the direct-weight GEMM when it applies. Returns 0 when it does
+// not, 1 when y was written, 2 when the two ranges' f32 partials were left in
+// `area` ([2][m][n], for the caller to add in order).
+uint32_t launch_q4_gemm_direct(hipStream_t stream, uint32_t cus, const uint16_t *x, uint32_t x_ld,
+                               const uint32_t *wq, const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t n,
+                               uint32_t k, void *y, int y_is_f32, void *area) {
+    const uint32_t tiles_m = (m + kDBM - 1) / kDBM, tiles_n = (n + kDBN - 1) / kDBN;
+    const uint64_t tiles = static_cast<uint64_t>(tiles_m) * tiles_n;
+    const uint32_t splits = direct_gemm_splits(cus, x_ld, m, n, k, area != nullptr);
+    if (splits == 0) return 0;
     direct_lds_opt_in();
     const uint32_t gm = xcd_rect_rows(tiles, tiles_m, tiles_n, k / splits);
     if (splits > 1) {

@@ -328,6 +328,31 @@ def test_gemm_split_k(device, oracle, m, n, k):
     run_linear(device, oracle, m, n, k, seed=5000 + m + n, sample=(64, n) if m > 64 else None)
 
 
+# The few-row kernel (q4_gemm_rows.hip): 1, 2 and 4 row tiles (edges at 16, 32
+# and 64 rows, two row blocks at 65), 1..7 column tiles per block with ragged
+# last tiles, one 128-value chunk for eight wavefronts, uneven chunk counts,
+# several scale/bias slots (k = 14336), the largest k its slots hold (32768)
+# and the first it leaves to the 256-row kernel (32896), and a row stride
+# above k. Same bound as every GEMM; a second run is bit-identical.
+@pytest.mark.parametrize("m,n,k,x_ld", [(9, 16, 128, 128), (17, 33, 384, 392), (33, 1000, 1152, 1152),
+                                        (64, 4100, 1152, 1160), (65, 5120, 768, 768), (12, 20470, 256, 256),
+                                        (24, 24570, 256, 256), (40, 10250, 512, 512), (16, 28664, 640, 640),
+                                        (32, 28672, 512, 512), (64, 16376, 640, 640), (64, 28650, 128, 128),
+                                        (100, 130, 14336, 14336), (9, 16, 32768, 32768), (9, 16, 32896, 32896)])
+def test_gemm_few_rows(device, oracle, m, n, k, x_ld):
+    seed = 11000 + m + n + k
+    wq, s, b = synth.q4_weights(seed, n, k)
+    x = synth.bf16_normal(seed + 1, (m, x_ld))
+    w = weight(device, wq, s, b)
+    xt = up(device, x, DType.BF16)
+    y32 = matmul_raw(device, xt, w, m, k, x_ld, _lib.F32)
+    y16 = matmul_raw(device, xt, w, m, k, x_ld, _lib.BF16)
+    again = matmul_raw(device, xt, w, m, k, x_ld, _lib.F32)
+    assert np.array_equal(y32.view(np.uint32), again.view(np.uint32)), "sums differ between runs"
+    y64 = oracle.linear_f64(np.ascontiguousarray(x[:, :k]), wq, s, b)
+    check_matmul(y32, y16, y64)
+
+
 def test_gemm_golden(device):
     with np.load(GOLDEN) as g:
         w = weight(device, g["gemm_wq"], g["gemm_s"], g["gemm_b"])
