@@ -5,10 +5,13 @@
 // index_select, cat and slice_scatter, each over strided views.
 //
 // These are plain kernels, one output element per thread (one block per
-// output element for the reductions), with the Metal kernels' arithmetic:
+// output element for the reductions; the matmul on the fp32 matrix cores),
+// with the Metal kernels' arithmetic:
 // values decoded to fp32, the op in fp32, one rounding on the way out
 // (src/metal/kernels/common.metal:29-43). They serve the model code that
 // runs op by op; the decoder's hot path has its own fused kernels.
+#include <type_traits>
+
 #include "device.hpp"
 #include "q4_common.hpp"
 
@@ -174,28 +177,149 @@ __global__ __launch_bounds__(kThreads) void argmax_kernel(const typename Float<D
     }
 }
 
-// Batched matmul over strided operands. A block owns a 32 x 32 output tile
-// of one batch entry; 256 threads each hold 2 x 2 sums. Operand tiles of 16
-// along k go through LDS as fp32; every sum runs over k in order (one fma per
-// step), as matmul_tiled accumulates (src/metal/kernels/matmul.metal:42-64).
+// Batched matmul over strided operands on the matrix cores, in fp32:
+// v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one fma at
+// a time in order of k, so every sum is the chain of fmas over k that
+// matmul_tiled forms (src/metal/kernels/matmul.metal:42-64); checked bit for
+// bit on the GPU against fmaf for 1M sums of normal, huge, tiny, denormal,
+// infinite and NaN values.
+// A block of four wavefronts (WM x WN) owns WM * 16 T rows x WN * 16 T columns
+// of one batch entry; operand tiles of 32 along k go through LDS as fp32, the
+// next tile's global loads in flight while one is computed. In LDS a row's (or
+// column's) 32 values lie by k % 4, then k / 4, 8 together: a lane's operands
+// of 8 MFMAs are two conflict-free 16-byte reads. Values past k are filled
+// with +0 (lhs) and -0 (rhs), whose product leaves every sum as it is.
+// Bounded by the fp32 matrix-core rate (157 TFLOP/s). Before, a thread kept
+// 2 x 2 sums fed by scalar LDS reads. bf16, before and now: 24 x [512, 128] x
+// [128, 512] (keys transposed in place) 69.2 -> 26.5 us, 24 x [512, 512] x
+// [512, 128] 73.9 -> 34.2 us, [16, 3072] x [3072, 8192] 224.6 -> 74.4 us.
 struct MatmulShape {
     uint32_t m, n, k, batch_ndim;
     uint32_t batch_dims[2];
     int64_t l_off, l_rs, l_cs, l_bs[2];
     int64_t r_off, r_rs, r_cs, r_bs[2];
+    int l_mode, r_mode;  // Stage
 };
 
-constexpr uint32_t kMmTile = 32;
-constexpr uint32_t kMmK = 16;
+constexpr uint32_t kMmK = 32;
+constexpr uint32_t kMmPitch = kMmK + 4;
 
+// How an operand's tile is read: single values with threads along k or along
+// the rows, or 8 values at once where the dim is contiguous, its extent a
+// multiple of 8 and every piece 16-byte aligned.
+enum Stage { kAlongK, kAlongRows, kPiecesK, kPiecesRows };
+
+typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+
+// 8 consecutive values from 16-byte aligned memory.
 template <int DT>
+__device__ __forceinline__ void load8(const typename Float<DT>::T *p, float (&v)[8]) {
+    if constexpr (DT == FH_BF16) {
+        const uint4 u = *reinterpret_cast<const uint4 *>(p);
+        const uint32_t w[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v[2 * e] = __uint_as_float(w[e] << 16);
+            v[2 * e + 1] = __uint_as_float(w[e] & 0xFFFF0000u);
+        }
+    } else {
+        const float4 lo = *reinterpret_cast<const float4 *>(p), hi = *reinterpret_cast<const float4 *>(p + 4);
+        v[0] = lo.x, v[1] = lo.y, v[2] = lo.z, v[3] = lo.w;
+        v[4] = hi.x, v[5] = hi.y, v[6] = hi.z, v[7] = hi.w;
+    }
+}
+
+// One operand's R x 32 tile on its way from memory to LDS: R * 4 pieces of 8
+// values over the block's threads. PIECES: the mode is one of the two that
+// read 8 values at once (the gathers' addresses cost the kernel 60 registers).
+template <int DT, int R, bool PIECES>
+struct MmTile {
+    using T = typename Float<DT>::T;
+    static constexpr int kItems = (R * 4 + static_cast<int>(kThreads) - 1) / static_cast<int>(kThreads);
+    static constexpr int kSingles = R * static_cast<int>(kMmK) / static_cast<int>(kThreads);
+    static_assert(kSingles <= kItems * 8, "single values fit the pieces' registers");
+    float v[kItems * 8];
+
+    // Row and first k of a piece, or row and k of a single value.
+    __device__ static void piece(int mode, uint32_t item, uint32_t *r, uint32_t *kk) {
+        if (mode == kPiecesK)
+            *r = item / 4, *kk = item % 4 * 8;
+        else
+            *kk = item / (R / 8), *r = item % (R / 8) * 8;
+    }
+    __device__ static void single(int mode, uint32_t i, uint32_t *r, uint32_t *kk) {
+        if (mode == kAlongK)
+            *r = i / kMmK, *kk = i % kMmK;
+        else
+            *kk = i / R, *r = i % R;
+    }
+    __device__ void load(const T *p, int64_t base, int64_t rs, int64_t ks, uint32_t row0, uint32_t rows, uint32_t k0,
+                         uint32_t k, int mode, float fill) {
+        uint32_t r, kk;
+        if (PIECES || mode >= kPiecesK) {
+#pragma unroll
+            for (int i = 0; i < kItems; ++i) {
+                const uint32_t item = threadIdx.x + i * kThreads;
+                if (R * 4 % kThreads != 0 && item >= R * 4) break;
+                piece(mode, item, &r, &kk);
+                // the extents are multiples of 8: a piece is inside or outside
+                float(&o)[8] = *reinterpret_cast<float(*)[8]>(v + i * 8);
+                if (row0 + r < rows && k0 + kk < k)
+                    load8<DT>(p + base + static_cast<int64_t>(row0 + r) * rs + static_cast<int64_t>(k0 + kk) * ks, o);
+                else
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) o[e] = fill;
+            }
+            return;
+        }
+        // requested without a branch each (a value outside reads the first)
+#pragma unroll
+        for (int e = 0; e < kSingles; ++e) {
+            single(mode, threadIdx.x + e * kThreads, &r, &kk);
+            const bool in = row0 + r < rows && k0 + kk < k;
+            const int64_t at = base + static_cast<int64_t>(row0 + r) * rs + static_cast<int64_t>(k0 + kk) * ks;
+            const float x = Float<DT>::get(p, in ? at : base);
+            v[e] = in ? x : fill;
+        }
+    }
+    __device__ void store(float *lds, int mode) const {
+        uint32_t r, kk;
+        if (!PIECES && mode < kPiecesK) {
+#pragma unroll
+            for (int e = 0; e < kSingles; ++e) {
+                single(mode, threadIdx.x + e * kThreads, &r, &kk);
+                lds[r * kMmPitch + kk % 4 * 8 + kk / 4] = v[e];
+            }
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < kItems; ++i) {
+            const uint32_t item = threadIdx.x + i * kThreads;
+            if (R * 4 % kThreads != 0 && item >= R * 4) break;
+            piece(mode, item, &r, &kk);
+            const float *const o = v + i * 8;
+            if (mode == kPiecesK) {
+                float *d = lds + r * kMmPitch + kk / 4;  // k % 4 = 0..3, k / 4 and k / 4 + 1
+#pragma unroll
+                for (int q = 0; q < 4; ++q) *reinterpret_cast<float2 *>(d + q * 8) = make_float2(o[q], o[q + 4]);
+            } else {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) lds[(r + e) * kMmPitch + kk % 4 * 8 + kk / 4] = o[e];
+            }
+        }
+    }
+};
+
+template <int DT, int WM, int WN, int T, bool PIECES>
 __global__ __launch_bounds__(kThreads) void matmul_kernel(const typename Float<DT>::T *__restrict__ lhs,
                                                           const typename Float<DT>::T *__restrict__ rhs, MatmulShape s,
                                                           typename Float<DT>::T *__restrict__ dst) {
-    __shared__ float lt[kMmTile][kMmK + 1];
-    __shared__ float rt[kMmK][kMmTile + 1];
-    const uint32_t t = threadIdx.x;
-    const uint32_t row0 = blockIdx.y * kMmTile, col0 = blockIdx.x * kMmTile;
+    constexpr int kBM = WM * 16 * T, kBN = WN * 16 * T;
+    static_assert(WM * WN * 64 == static_cast<int>(kThreads), "four wavefronts");
+    __shared__ __attribute__((aligned(16))) float lt[kBM * kMmPitch];
+    __shared__ __attribute__((aligned(16))) float rt[kBN * kMmPitch];
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t row0 = blockIdx.y * kBM, col0 = blockIdx.x * kBN;
     // batch entry -> each operand's base offset (batch dims row-major)
     int64_t lb = s.l_off, rb = s.r_off;
     uint32_t b = blockIdx.z;
@@ -205,37 +329,103 @@ __global__ __launch_bounds__(kThreads) void matmul_kernel(const typename Float<D
         rb += static_cast<int64_t>(b % size) * s.r_bs[d];
         b /= size;
     }
-    const uint32_t tr = (t / 16) * 2, tc = (t % 16) * 2;  // this thread's 2 x 2 sums
-    float acc[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+    f32x4_t acc[T][T];
+#pragma unroll
+    for (int i = 0; i < T; ++i)
+#pragma unroll
+        for (int j = 0; j < T; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][r] = 0.f;
+    MmTile<DT, kBM, PIECES> lv;
+    MmTile<DT, kBN, PIECES> rv;
+    const float *const la = lt + ((wave / WN) * 16 * T + (lane & 15)) * kMmPitch + (lane >> 4) * 8;
+    const float *const ra = rt + ((wave % WN) * 16 * T + (lane & 15)) * kMmPitch + (lane >> 4) * 8;
+    if (s.k > 0) {
+        lv.load(lhs, lb, s.l_rs, s.l_cs, row0, s.m, 0, s.k, s.l_mode, 0.f);
+        rv.load(rhs, rb, s.r_cs, s.r_rs, col0, s.n, 0, s.k, s.r_mode, -0.f);
+    }
     for (uint32_t k0 = 0; k0 < s.k; k0 += kMmK) {
-        // 32 x 16 of lhs and 16 x 32 of rhs: two loads per thread each
-        for (uint32_t e = t; e < kMmTile * kMmK; e += kThreads) {
-            const uint32_t r = e / kMmK, kk = e % kMmK;
-            const uint32_t gr = row0 + r, gk = k0 + kk;
-            lt[r][kk] = (gr < s.m && gk < s.k) ? Float<DT>::get(lhs, lb + gr * s.l_rs + gk * s.l_cs) : 0.0f;
-            const uint32_t kr = e / kMmTile, c = e % kMmTile;
-            const uint32_t rk = k0 + kr, gc = col0 + c;
-            rt[kr][c] = (rk < s.k && gc < s.n) ? Float<DT>::get(rhs, rb + rk * s.r_rs + gc * s.r_cs) : 0.0f;
-        }
+        __syncthreads();  // the previous tile's reads are done
+        lv.store(lt, s.l_mode);
+        rv.store(rt, s.r_mode);
         __syncthreads();
-        const uint32_t steps = s.k - k0 < kMmK ? s.k - k0 : kMmK;
-        for (uint32_t kk = 0; kk < steps; ++kk) {
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = fmaf(lt[tr + i][kk], rt[kk][tc + j], acc[i][j]);
+        if (k0 + kMmK < s.k) {
+            lv.load(lhs, lb, s.l_rs, s.l_cs, row0, s.m, k0 + kMmK, s.k, s.l_mode, 0.f);
+            rv.load(rhs, rb, s.r_cs, s.r_rs, col0, s.n, k0 + kMmK, s.k, s.r_mode, -0.f);
         }
-        __syncthreads();
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            f32x4_t a[T], c[T];
+#pragma unroll
+            for (int i = 0; i < T; ++i) a[i] = *reinterpret_cast<const f32x4_t *>(la + i * 16 * kMmPitch + h * 4);
+#pragma unroll
+            for (int j = 0; j < T; ++j) c[j] = *reinterpret_cast<const f32x4_t *>(ra + j * 16 * kMmPitch + h * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < T; ++i)
+#pragma unroll
+                    for (int j = 0; j < T; ++j)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i][e], c[j][e], acc[i][j], 0, 0, 0);
+        }
     }
     const uint64_t out_base = static_cast<uint64_t>(blockIdx.z) * s.m * s.n;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < T; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const uint32_t r = row0 + tr + i, c = col0 + tc + j;
-            if (r < s.m && c < s.n) Float<DT>::put(dst, static_cast<int64_t>(out_base + static_cast<uint64_t>(r) * s.n + c),
-                                                 acc[i][j]);
-        }
+        for (int j = 0; j < T; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const uint32_t row = row0 + ((wave / WN) * T + i) * 16 + 4 * (lane >> 4) + r;
+                const uint32_t col = col0 + ((wave % WN) * T + j) * 16 + (lane & 15);
+                if (row < s.m && col < s.n)
+                    Float<DT>::put(dst, static_cast<int64_t>(out_base + static_cast<uint64_t>(row) * s.n + col),
+                                   acc[i][j][r]);
+            }
+}
+
+// How an operand's tile is read: rs, ks its strides along the rows (columns
+// for rhs) and k, `base` the address of its first element.
+int stage_mode(const void *base, int size, int64_t rs, int64_t ks, int64_t rows, int64_t k, const int64_t *bs,
+               uint32_t batch_ndim) {
+    bool pieces = reinterpret_cast<uintptr_t>(base) % 16 == 0;  // and every batch entry's first element
+    const int64_t per = 16 / size;                              // elements in 16 bytes
+    for (uint32_t d = 0; d < batch_ndim; ++d) pieces = pieces && bs[d] % per == 0;
+    if (pieces && ks == 1 && k % 8 == 0 && (rs % per == 0 || rows == 1)) return kPiecesK;
+    if (pieces && rs == 1 && rows % 8 == 0 && (ks % per == 0 || k == 1)) return kPiecesRows;
+    return ks <= rs ? kAlongK : kAlongRows;
+}
+
+// Launches the tile for the shape: 64 x 64 outputs a block; 32 x 128 or 128 x
+// 32 where one extent is at most 32; 32 x 32 (a quarter of the sums a
+// wavefront) where the larger ones would give fewer blocks than CUs (24 x
+// [512, 512] x [512, 128], 384 blocks of 64 x 64: 43 us against 64 us in 1536
+// of 32 x 32).
+template <int DT>
+void launch_matmul(hipStream_t stream, uint32_t cus, const void *lhs, const void *rhs, const MatmulShape &s,
+                   uint32_t batch, void *dst) {
+    using E = typename Float<DT>::T;
+    auto go = [&](auto kernel, uint32_t bm, uint32_t bn) {
+        hipLaunchKernelGGL(kernel, dim3((s.n + bn - 1) / bn, (s.m + bm - 1) / bm, batch), dim3(kThreads), 0, stream,
+                           static_cast<const E *>(lhs), static_cast<const E *>(rhs), s, static_cast<E *>(dst));
+    };
+    const uint32_t bm = s.m <= 32 ? 32 : s.n <= 32 ? 128 : 64, bn = s.m <= 32 ? 128 : s.n <= 32 ? 32 : 64;
+    const uint64_t blocks = static_cast<uint64_t>((s.m + bm - 1) / bm) * ((s.n + bn - 1) / bn) * batch;
+    auto pick = [&](auto pieces) {
+        constexpr bool P = decltype(pieces)::value;
+        if (blocks < cus)
+            go(matmul_kernel<DT, 2, 2, 1, P>, 32, 32);
+        else if (bm == 32)
+            go(matmul_kernel<DT, 1, 4, 2, P>, 32, 128);
+        else if (bn == 32)
+            go(matmul_kernel<DT, 4, 1, 2, P>, 128, 32);
+        else
+            go(matmul_kernel<DT, 2, 2, 2, P>, 64, 64);
+    };
+    if (s.l_mode >= kPiecesK && s.r_mode >= kPiecesK)
+        pick(std::true_type{});
+    else
+        pick(std::false_type{});
 }
 
 // index_select_rows (src/metal/kernels/index_select.metal:11-29): an id at
@@ -560,20 +750,21 @@ extern "C" int fh_matmul(fh_device *dev, int dtype, const void *lhs, const fh_vi
     if (batch > 65535) return fail(FH_ERR_INDEX_TOO_LARGE, "%s: %lld batch entries exceed the grid", fn,
                                    (long long)batch);
     if (int rc = set_current(dev, fn)) return rc;
-    const dim3 grid((s.n + kMmTile - 1) / kMmTile, (s.m + kMmTile - 1) / kMmTile, static_cast<uint32_t>(batch));
-    if (grid.y > 65535) return fail(FH_ERR_INDEX_TOO_LARGE, "%s: m=%u exceeds the grid", fn, s.m);
-    // grid.x * 256 work-items must stay below 2^32
-    if (static_cast<uint64_t>(grid.x) * kThreads > 0xFFFFFFFFull)
+    // the limits of a grid of 32 x 32 tiles: rows in grid.y, and grid.x * 256
+    // work-items below 2^32
+    if ((s.m + 31) / 32 > 65535) return fail(FH_ERR_INDEX_TOO_LARGE, "%s: m=%u exceeds the grid", fn, s.m);
+    if (static_cast<uint64_t>((s.n + 31) / 32) * kThreads > 0xFFFFFFFFull)
         return fail(FH_ERR_INDEX_TOO_LARGE, "%s: n=%u exceeds the grid", fn, s.n);
+    const int size = itemsize(dtype);
+    s.l_mode = stage_mode(static_cast<const char *>(lhs) + s.l_off * size, size, s.l_rs, s.l_cs, s.m, s.k, s.l_bs,
+                          s.batch_ndim);
+    s.r_mode = stage_mode(static_cast<const char *>(rhs) + s.r_off * size, size, s.r_cs, s.r_rs, s.n, s.k, s.r_bs,
+                          s.batch_ndim);
     return dispatch(dev, fn, [&] {
         if (dtype == FH_F32)
-            hipLaunchKernelGGL(matmul_kernel<FH_F32>, grid, dim3(kThreads), 0, dev->stream,
-                               static_cast<const float *>(lhs), static_cast<const float *>(rhs), s,
-                               static_cast<float *>(dst));
+            launch_matmul<FH_F32>(dev->stream, dev->compute_units, lhs, rhs, s, static_cast<uint32_t>(batch), dst);
         else
-            hipLaunchKernelGGL(matmul_kernel<FH_BF16>, grid, dim3(kThreads), 0, dev->stream,
-                               static_cast<const uint16_t *>(lhs), static_cast<const uint16_t *>(rhs), s,
-                               static_cast<uint16_t *>(dst));
+            launch_matmul<FH_BF16>(dev->stream, dev->compute_units, lhs, rhs, s, static_cast<uint32_t>(batch), dst);
     });
 }
 

@@ -385,6 +385,48 @@ def test_matmul_on_strided_batches(device, dtype):
     assert np.all(np.abs(got - want) <= bound)
 
 
+# (batch, m, k, n): one value; tiles cut at every edge; a k tail; and, with at
+# least one block per CU, each larger tile (64 x 64, 32 x 128, 128 x 32)
+MATMUL_SHAPES = [(1, 1, 1, 1), (1, 33, 31, 65), (3, 64, 32, 64), (2, 40, 96, 72), (12, 296, 40, 304),
+                 (4, 20, 33, 8320), (4, 8320, 24, 20)]
+
+
+@pytest.mark.parametrize("dtype", [DType.F32, DType.BF16])
+@pytest.mark.parametrize("batch,m,k,n", MATMUL_SHAPES)
+def test_matmul_sums_are_the_chain_over_k(device, dtype, batch, m, k, n):
+    """Every sum is one fma per k in order, whatever the tile and however the
+    operands are read: contiguous, transposed (pieces along either dim),
+    offset by one element (no aligned pieces), broadcast over the batch. The
+    values have 8-bit significands, so a * b is exact in float32 and the
+    chain is float32 additions: compared bit for bit."""
+    rng = np.random.default_rng(batch + m + k + n)
+    bits = lambda a: (R.rne(a).view(np.uint32) >> 16).astype(np.uint16)
+    bf = lambda a: R.from_bf16(bits(a.astype(np.float32)))
+
+    def operand(rows, cols, how):
+        """[batch, rows, cols] values and a tensor of them read as `how`."""
+        a = bf(rng.standard_normal((1 if how == "broadcast" else batch, rows, cols)))
+        store = np.swapaxes(a, 1, 2) if how == "transposed" else a
+        flat = np.concatenate([np.zeros(1 if how == "offset" else 0, np.float32), store.ravel()])
+        t = f32(device, flat, (flat.size,)).to_dtype(device, dtype).narrow(0, flat.size - store.size, store.size)
+        t = t.reshape(store.shape)
+        t = t.permute((0, 2, 1)) if how == "transposed" else t.expand((batch, rows, cols))
+        return np.broadcast_to(a, (batch, rows, cols)), t
+
+    big = batch * m * n > 1 << 20
+    for lhow, rhow in (("plain", "transposed"), ("transposed", "plain"), ("offset", "offset"), ("broadcast", "plain")):
+        if big and lhow == "offset":
+            continue
+        ln, lt = operand(m, k, lhow)
+        rn, rt = operand(k, n, rhow)
+        want = np.zeros((batch, m, n), np.float32)
+        for kk in range(k):
+            want += ln[:, :, kk:kk + 1] * rn[:, kk:kk + 1, :]
+        got = lt.matmul(device, rt).to_numpy(device)
+        exact = bits(want) if dtype is DType.BF16 else want.view(np.uint32)
+        assert np.array_equal(got.view(exact.dtype), exact), (lhow, rhow)
+
+
 def test_strided_entry_points_reject_bad_views(device):
     """Out-of-allocation views and mismatched dims are refused on the host."""
     import ctypes
