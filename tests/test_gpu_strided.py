@@ -23,7 +23,7 @@ import pytest
 
 from foundry_amd import _lib
 from foundry_amd.device import HipDevice
-from foundry_amd.primitive import DType, TensorError
+from foundry_amd.primitive import Copy, DType, TensorError
 from foundry_amd.tensor import Tensor
 from oracle import llama_ref as R
 
@@ -383,6 +383,66 @@ def test_matmul_on_strided_batches(device, dtype):
     if dtype is DType.BF16:
         bound = bound + 2.0 ** -8 * np.abs(want)
     assert np.all(np.abs(got - want) <= bound)
+
+
+# Shapes whose walks merge to one dim or none, with last dims that are and are
+# not whole 16-byte pieces, more than a block of either, and one element
+WALK_SHAPES = [(1,), (7,), (8,), (3, 1, 5, 8), (2, 3, 4, 16), (4, 1000), (2, 513, 24), (5, 7, 11, 13)]
+
+
+@pytest.mark.parametrize("dtype", [DType.F32, DType.BF16])
+@pytest.mark.parametrize("shape", WALK_SHAPES)
+def test_elementwise_and_moves_over_every_walk(device, dtype, shape):
+    """add, neg, copy, to_dtype, cat and slice_scatter over contiguous views,
+    views one element off 16-byte alignment, permuted ones and ones broadcast
+    along the first or last dim: bit for bit what numpy gives."""
+    rng = np.random.default_rng(sum(shape))
+
+    def operand(how):
+        dims = list(shape)
+        if how == "first":
+            dims[0] = 1
+        if how == "last":
+            dims[-1] = 1
+        order = tuple(reversed(range(len(shape))))
+        a = _as_dtype(rng.standard_normal(dims).astype(np.float32), dtype)
+        flat = (a.transpose(order) if how == "permuted" else a).ravel()
+        off = 1 if how == "offset" else 0
+        t = f32(device, np.concatenate([np.zeros(off, np.float32), flat]), (flat.size + off,)).to_dtype(device, dtype)
+        t = t.narrow(0, off, flat.size).reshape([dims[d] for d in order] if how == "permuted" else dims)
+        return (t.permute(order) if how == "permuted" else t).expand(shape), np.broadcast_to(a, shape)
+
+    bits = lambda a, dt: (a.view(np.uint32) >> 16).astype(np.uint16) if dt is DType.BF16 else a.view(np.uint32)
+    same = lambda t, want: np.array_equal(t.to_numpy(device).view(np.uint16 if t.dtype is DType.BF16 else np.uint32),
+                                          bits(_as_dtype(np.ascontiguousarray(want), t.dtype), t.dtype))
+    plain, pn = operand("plain")
+    for how in ("plain", "offset", "permuted", "first", "last"):
+        t, tn = operand(how)
+        assert same(plain.add(device, t), pn + tn) and same(t.add(device, plain), pn + tn), how
+        assert same(t.neg(device), -tn), how
+        assert same(t.apply(device, Copy(), []), tn), how
+        assert same(t.to_dtype(device, DType.F32 if dtype is DType.BF16 else DType.BF16), tn), how
+        assert same(Tensor.cat(device, [t, plain], 0), np.concatenate([tn, pn])), how
+        target = Tensor.zeros(device, dtype, (shape[0] + 3, *shape[1:]))
+        target.slice_scatter(device, t, 0, 2)
+        want = np.zeros((shape[0] + 3, *shape[1:]), np.float32)
+        want[2:2 + shape[0]] = tn
+        assert same(target, want), how
+
+
+@pytest.mark.parametrize("dtype", [DType.F32, DType.BF16])
+@pytest.mark.parametrize("size", [1, 63, 64, 65, 192, 255, 256, 257, 700])
+def test_reductions_of_many_rows(device, dtype, size):
+    """At least 16 rows per CU are reduced a wavefront per row, in the order of
+    the 256-thread fold and tree all the same; along the last dim and a
+    strided one."""
+    rng = np.random.default_rng(size)
+    an = _as_dtype(rng.standard_normal((8200, size)).astype(np.float32), dtype)
+    for t, dim in ((f32(device, an, an.shape), 1), (f32(device, an.T, an.T.shape), 0)):
+        t = t.to_dtype(device, dtype)
+        s, m = values(device, t.sum_keepdim(device, dim)), values(device, t.amax_keepdim(device, dim))
+        assert np.array_equal(s.ravel(), _as_dtype(_reduce_restated(an, False), dtype)), dim
+        assert np.array_equal(m.ravel(), _as_dtype(_reduce_restated(an, True), dtype)), dim
 
 
 # (batch, m, k, n): one value; tiles cut at every edge; a k tail; and, with at
