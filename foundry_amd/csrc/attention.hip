@@ -48,7 +48,10 @@
 // its KV head's keys itself (16 wavefronts, a chunk each), meets the chunks'
 // statistics at block barriers and sums P.V for a 16-dim slice of V. Its
 // cost is the keys every block pulls through one CU (about 34 GB/s per CU
-// in the matrix-core fragment pattern), so it only pays for short caches.
+// in the matrix-core fragment pattern), so it only pays for short caches,
+// and only while its blocks all run at once (launch_decode_short).
+#include <atomic>
+
 #include "decoder_common.hpp"
 #include "q4_gemv_mfma.hpp"
 
@@ -98,9 +101,15 @@ struct AttnLayout {
 
 constexpr int kPvTile = 64;  // keys per tile of the chunked P.V
 // The sliced P.V reads V in 4-byte pieces (a 16-dim slice of a key row is 32
-// bytes): below this many keys per (row, KV head) pair, summed over the
-// launch, it still wins by skipping the combine pass.
+// bytes), and each block walks all of its row's keys: it still wins, by
+// skipping the combine pass, for caches shorter than kPvChunkedMinLen with
+// fewer than kPvChunkedMinKeys keys summed over the launch's (row, KV head)
+// pairs. Decode attention, 8 KV heads of 128, sliced against chunked: one row
+// 8.7 / 10.7 us at 200 positions, 10.4 / 10.9 at 350, 11.0 / 10.9 at 500, 13.0
+// / 10.9 at 768, 16.7 / 11.1 at 1100, 22.9 / 11.4 at 2000; 8 rows 10.2 / 11.4
+// at 200.
 constexpr uint64_t kPvChunkedMinKeys = FH_PV_CHUNKED_MIN_KEYS;
+constexpr uint64_t kPvChunkedMinLen = 448;
 
 static AttnLayout attn_layout(uint64_t rows, uint64_t n_heads, uint64_t n_kv, uint64_t head_dim,
                               uint64_t max_len) {
@@ -116,7 +125,7 @@ static AttnLayout attn_layout(uint64_t rows, uint64_t n_heads, uint64_t n_kv, ui
     a.scores = round_up(rows * n_heads * a.nck * 8);
     a.part = a.scores + round_up(rows * n_heads * max_len * 2);
     a.chunks = a.chunk_keys = 0;
-    if (blocks * max_len >= kPvChunkedMinKeys) {
+    if (blocks * max_len >= kPvChunkedMinKeys || max_len >= kPvChunkedMinLen) {
         const uint64_t tiles = (max_len + kPvTile - 1) / kPvTile;
         const uint64_t want_pv = blocks ? (kPvTargetBlocks + blocks - 1) / blocks : 1;
         uint64_t chunks = want_pv < tiles ? want_pv : tiles;
@@ -1354,8 +1363,8 @@ static bool launch_attention_shape(int64_t head_dim, int64_t g, hipStream_t stre
     return false;
 }
 
-// Caches of at most this many positions take attn_decode_short_kernel
-// (head_dim 64 or 128).
+// Caches of at most this many positions may take attn_decode_short_kernel
+// (head_dim 64 or 128; launch_decode_short says when).
 #ifndef FH_DECODE_SHORT_MAX_LEN
 #define FH_DECODE_SHORT_MAX_LEN 1024
 #endif
@@ -1367,8 +1376,15 @@ static_assert(kDecodeShortMaxLen <= kShortKeys, "one chunk per wavefront");
 #endif
 constexpr int kShortDims = FH_DECODE_SHORT_DIMS;  // V dims per block
 
+// Launches the one-launch kernel where its blocks, n_kv * HD / kShortDims per
+// row and a wavefront per chunk, run at once or nearly (up to a third of a
+// second round); false otherwise. In more rounds every block pulls its head's
+// keys through a CU again, which the split form does not: 8 rows of 8 KV heads
+// of 128, 1000 positions, 74.8 us against 15.7 us split; 2 rows at 768 16.3 /
+// 11.2; on the other side 2 rows at 500 9.8 / 11.1, one row at 1000 11.0 /
+// 11.1, and 8 rows of heads of 64 at 500 (a round and a third) 12.6 / 13.5.
 template <int HD, int G>
-static void launch_decode_short(hipStream_t stream, uint32_t rows, const AttnArgs &x) {
+static bool launch_decode_short(hipStream_t stream, uint32_t cus, uint32_t rows, const AttnArgs &x) {
     // one wavefront per 64-key chunk the cache can hold (positions beyond
     // max_len take no chunk), and at least the RoPE and value lanes
     const uint32_t chunk_waves = (x.max_len + kAttnChunk - 1) / kAttnChunk;
@@ -1377,18 +1393,31 @@ static void launch_decode_short(hipStream_t stream, uint32_t rows, const AttnArg
     const uint32_t out_waves = (G * kShortDims + 63) / 64;
     uint32_t waves = chunk_waves > rope_waves ? chunk_waves : rope_waves;
     if (out_waves > waves) waves = out_waves;
+    // resident blocks per CU by block size, asked of the runtime once each
+    static std::atomic<int> resident[kShortWaves + 1];
+    int per_cu = resident[waves].load(std::memory_order_relaxed);
+    if (per_cu == 0) {
+        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, attn_decode_short_kernel<HD, G, kShortDims>,
+                                                         static_cast<int>(64 * waves), 0) != hipSuccess ||
+            per_cu < 1) {
+            (void)hipGetLastError();
+            per_cu = 1;
+        }
+        resident[waves].store(per_cu, std::memory_order_relaxed);
+    }
     const dim3 grid(x.n_kv * (HD / kShortDims), rows);
+    if (3ull * grid.x * rows > 4ull * cus * static_cast<uint64_t>(per_cu)) return false;
     hipLaunchKernelGGL((attn_decode_short_kernel<HD, G, kShortDims>), grid, dim3(64 * waves), 0, stream, x.q_src, x.cos_tab,
                        x.sin_tab, x.positions, x.pos_limit, x.k_cache, x.v_cache, x.row_stride, x.n_heads, x.n_kv,
                        x.max_len, x.scale, x.out);
+    return true;
 }
 
-static bool launch_decode_short_shape(int64_t head_dim, int64_t g, hipStream_t stream, uint32_t rows,
+static bool launch_decode_short_shape(int64_t head_dim, int64_t g, hipStream_t stream, uint32_t cus, uint32_t rows,
                                       const AttnArgs &x) {
 #define FH_SHORT_G(HD, GG)                                         \
     case GG:                                                       \
-        launch_decode_short<HD, GG>(stream, rows, x);              \
-        return true;
+        return launch_decode_short<HD, GG>(stream, cus, rows, x);
 #define FH_SHORT_HD(HD)                                            \
     if (head_dim == HD) switch (g) {                               \
             FH_SHORT_G(HD, 1)                                      \
@@ -1598,7 +1627,8 @@ int decode_attention(const char *fn, fh_device *dev, const uint16_t *qkv, int64_
     bool combined = false;
     const int rc = dispatch(dev, fn, [&] {
         if (!short_cache ||
-            !launch_decode_short_shape(head_dim, n_heads / n_kv, dev->stream, static_cast<uint32_t>(batch), x))
+            !launch_decode_short_shape(head_dim, n_heads / n_kv, dev->stream, dev->compute_units,
+                                       static_cast<uint32_t>(batch), x))
             combined = launch_attention_shape<true>(head_dim, n_heads / n_kv, dev->stream,
                                                     static_cast<uint32_t>(batch), a, x) &&
                        a.chunks > 1;

@@ -361,8 +361,8 @@ int fh_decode_attention_workspace(int64_t batch, int64_t n_heads, int64_t n_kv, 
 /* The decode step's attention for a batch of sequences that each add one
  * token: fh_rope_kv's RoPE of the token's q and k and its cache write at
  * positions[b], then fh_attention over keys 0..positions[b] of sequence b --
- * the same rounding points, in two kernel launches instead of three, or in
- * one when max_len <= 1024 and head_dim is 64 or 128 (the workspace is then
+ * the same rounding points, in two or three kernel launches, or in one for
+ * few rows with max_len <= 1024 and head_dim 64 or 128 (the workspace is then
  * not touched, but is still checked and required). qkv:
  * [batch, (n_heads + 2 n_kv) * head_dim]; cos_tab/sin_tab: [table_len,
  * head_dim]; positions: device u32 [batch]; k_cache/v_cache: batch x n_kv

@@ -308,6 +308,21 @@ def test_decode_attention(device, n_heads, n_kv, hd, batch, max_len):
         assert_attention_close(got[b:b + 1], ref, flip, (b, p))
 
 
+# Both sides of the rules that pick the decode form: caches of at most 1024
+# positions whose one-launch blocks run at once (8 rows of 8 heads of 128 at
+# 100, of 64 at 500) or would take more rounds (the same at 200 and 1000, 3
+# rows at 350, 32 KV heads at 1000), and the sliced or chunked P.V on either
+# side of 448 positions (head_dim 256 never takes the one-launch form).
+DECODE_RULE_CASES = [(32, 8, 128, 8, 100), (32, 8, 64, 8, 500), (32, 8, 128, 8, 200), (32, 8, 128, 8, 1000),
+                     (24, 8, 128, 3, 350), (32, 32, 128, 1, 1000), (8, 2, 256, 1, 447), (8, 2, 256, 1, 448),
+                     (24, 8, 128, 1, 1100)]
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd,batch,max_len", DECODE_RULE_CASES)
+def test_decode_attention_forms(device, n_heads, n_kv, hd, batch, max_len):
+    test_decode_attention(device, n_heads, n_kv, hd, batch, max_len)
+
+
 def test_decode_attention_dirty_workspace(device):
     """The chunked decode P.V (8 sequences x 8 KV heads x 4096 keys) leaves
     f32 partials per chunk in the workspace for the combine pass, which reads
