@@ -34,10 +34,10 @@
 //       rows.
 //   fh_attention with head_dim 128 uses attn_pv_tile_kernel instead: the
 //   query-row tiles of the scores, P.V on the matrix cores (M and S combined
-//   over each row's chunks in another fixed order). A prompt-length call
-//   whose 256-pair query tiles fill half the device takes one launch of
-//   attn_flash_kernel instead (attention_flash.hip): both passes over the
-//   keys in one block per tile, no workspace.
+//   over each row's chunks in another fixed order). A prompt that is not
+//   short against its cache takes one launch of attn_flash_kernel instead
+//   (attention_flash.hip, attention_flash_splits): both passes over the keys
+//   in one block per tile, no workspace.
 //   Every output element is a sum in a fixed order, so results do not
 //   change from run to run.
 // splits and slices make rows * n_kv * (blocks per pair) about
@@ -1524,8 +1524,8 @@ extern "C" int fh_attention(fh_device *dev, const uint16_t *q, const uint16_t *k
                      const_cast<uint16_t *>(v_cache), 0, static_cast<uint32_t>(n_heads),
                      static_cast<uint32_t>(n_kv), static_cast<uint32_t>(max_len), scale,
                      static_cast<char *>(workspace), out};
-    // prompt-length calls that fill the device: the one-pass kernel
-    // (attention_flash.hip), which leaves the workspace untouched
+    // prompts: the one-pass kernel (attention_flash.hip), which leaves the
+    // workspace untouched
     return dispatch(dev, fn, [&] {
         if (!launch_attention_flash(dev->stream, dev->compute_units, q, positions, static_cast<uint32_t>(tokens),
                                     k_cache, v_cache, static_cast<uint32_t>(n_heads), static_cast<uint32_t>(n_kv),

@@ -1,14 +1,16 @@
 // Prefill attention in one pass per query tile, with the reference's
 // rounding points: the counterpart of scaled_dot_product_attention
 // (src/nn/attention.rs:23-60) under the causal mask (src/nn/masking.rs:11-32)
-// for head_dim 128. Scores s_j = RNE(q.k_j) * scale (fp32 dot products, bf16
-// rounding, fp32 scale), M = max_j s_j, S = sum_j exp(s_j - M), probabilities
+// for head_dim 64 and 128. Scores s_j = RNE(q.k_j) * scale (fp32 dot products,
+// bf16 rounding, fp32 scale), M = max_j s_j, S = sum_j exp(s_j - M), probabilities
 // p_j = RNE(exp(s_j - M) / S) -- from the row's GLOBAL max and sum, as the
 // reference rounds them before P.V -- and out = RNE(sum_j p_j v_j).
 //
 // Design for CDNA4: block (KV head, tile of 256 / G query rows), 8 wavefronts;
 // the tile's (row, head) pairs are the columns of the score tiles, 32 per
-// wavefront. The keys are walked twice, 64 at a time through LDS:
+// wavefront. (With few tiles the keys are split over 2 or 4 wavefronts
+// instead, and a block holds 128 or 64 pairs.) The keys are walked twice, 64
+// or 128 at a time through LDS:
 //   pass 1: S^T = K Q^T on the matrix cores (v_mfma_f32_32x32x16_bf16, the
 //     keys as A rows, the pairs' q as B columns held in registers for the
 //     whole block), so a lane holds 16 keys of ONE pair: the running max and
@@ -21,8 +23,9 @@
 //     same order, so each B fragment is one 16-byte read.
 // No scores or statistics leave the CU (the two-kernel path writes both
 // through a workspace), and every key and value is read from L2 once per
-// 256 (row, head) pairs. Every sum runs in a fixed order, so results do not
-// change from run to run.
+// block. What bounds it is VALU issue: about 21 instructions per score, of
+// which a wavefront issues one per 8 clocks and a SIMD one per 4.6. Every sum
+// runs in a fixed order, so results do not change from run to run.
 #include <type_traits>
 
 #include "decoder_common.hpp"
@@ -31,11 +34,22 @@ namespace fh {
 
 namespace {
 
-constexpr int kFlHd = 128;
 constexpr int kFlThreads = 512;
 constexpr int kFlWaves = kFlThreads / 64;
-constexpr int kFlKeys = 64;                       // keys per LDS block
-constexpr uint32_t kFlKBlock = kFlKeys * kFlHd;   // bf16 per K or V block
+constexpr int kFlKeys = 64;  // keys per LDS block
+
+// Shape of a block: head size, and over how many wavefronts KS the keys of a
+// (row, head) pair are split (1, 2 or 4; the block then holds 256 / KS pairs).
+template <int HD, int KS>
+struct FlCfg {
+    static constexpr int kPairGroups = kFlWaves / KS;      // wavefronts of 32 pairs each
+    static constexpr uint32_t kPairs = 32 * kPairGroups;
+    static constexpr int kBlocks = KS == 1 ? 1 : 2;        // LDS blocks of 64 keys per trip
+    static constexpr uint32_t kKeys = kFlKeys * kBlocks;   // keys per trip
+    static constexpr int kTiles = KS == 4 ? 1 : 2;         // 32-key tiles a wavefront takes of them
+    static constexpr uint32_t kBuf = kKeys * HD;           // bf16 per K or V buffer (two of each)
+    static constexpr uint32_t kLds = 4 * kBuf * 2;         // bytes
+};
 
 typedef __attribute__((ext_vector_type(8))) __bf16 fl_bf16x8_t;
 typedef __attribute__((ext_vector_type(16))) float fl_f32x16_t;
@@ -97,46 +111,66 @@ struct FlExp {
 
 }  // namespace
 
-// Block (KV head, sequence, query tile): rows r0 .. r0 + 256 / G - 1 of
-// sequence blockIdx.y (`rows` rows each, its cache seq_cache elements after
-// the previous one's; K tiled in groups of 16 keys, k_tile; V [max_len][128])
-// over its cache. positions[r]: the row's position; it attends keys 0 ..
-// min(pos, max_len - 1). Tiles go out last first: a prompt's later rows
-// attend more keys, and the longest blocks then start first.
-template <int G>
-__global__ __launch_bounds__(kFlThreads) void attn_flash_kernel(
+// Block (KV head, sequence, query tile): rows r0 .. r0 + QT - 1 (QT = pairs of
+// the block / G) of sequence blockIdx.y (`rows` rows each, its cache seq_cache
+// elements after the previous one's; K tiled in groups of 16 keys, k_tile; V
+// [max_len][HD]) over its cache. positions[r]: the row's position; it attends
+// keys 0 .. min(pos, max_len - 1). Tiles go out last first: a prompt's later
+// rows attend more keys, and the longest blocks then start first.
+// With KS > 1 wavefront w holds pairs 32 (w % (8 / KS)) .. + 31 and every KS-th
+// run of 64 (KS = 4: 32) keys; the splits' statistics, and at the end their
+// sums of P.V, meet in LDS and are added in split order. Two blocks share a CU
+// where their registers allow it (heads of 64, 128 of them a lane: 2048 rows
+// after 1024 108 us, 124 at 130 registers).
+template <int HD, int G, int KS>
+__global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_flash_kernel(
     const uint16_t *__restrict__ q, const uint32_t *__restrict__ positions, uint32_t rows,
     const uint16_t *__restrict__ k_cache, const uint16_t *__restrict__ v_cache, uint64_t seq_cache, uint32_t n_heads,
     uint32_t max_len, float scale, uint16_t *__restrict__ out) {
-    constexpr uint32_t QT = 256 / G;   // query rows per block
-    constexpr uint32_t LIVE = QT * G;  // (row, head) pairs of the block
-    // K blocks: [key][16 pieces of 8 dims], piece slot s of key k holding
-    // piece s ^ (k % 16); V^T blocks: [dim][64 key slots], 16-byte piece slot
-    // s of dim d holding piece s ^ ((d / 2) % 8). Both are conflict-free for
-    // the fragment reads below.
-    __shared__ __align__(16) uint16_t kls[2][kFlKBlock];
-    __shared__ __align__(16) uint16_t vls[2][kFlKBlock];
-    // the wavefronts' longest contexts, read before V^T buffer 1 is first written
-    uint32_t *const wmax = reinterpret_cast<uint32_t *>(&vls[1][0]);
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, h = lane >> 5;
+    using C = FlCfg<HD, KS>;
+    constexpr uint32_t QT = C::kPairs / G;  // query rows per block
+    constexpr uint32_t LIVE = QT * G;       // (row, head) pairs of the block
+    constexpr int QS = HD / 16;             // MFMA k steps of a score
+    constexpr int DT = HD / 32;             // 32-dim tiles of the output
+    constexpr uint32_t PP = HD / 8;         // 16-byte pieces per key
+    // K buffers: [key][PP pieces of 8 dims], piece slot s of key k holding
+    // piece s ^ swz(k); V^T buffers: blocks of [dim][64 key slots], 16-byte
+    // piece slot s of dim d holding piece s ^ ((d / 2) % 8). Both are
+    // conflict-free for the fragment reads below.
+    extern __shared__ __align__(16) uint16_t fl_smem[];
+    // set when V of a key that not every row attends is inf or NaN: such a
+    // value is staged as 0, since its probability of 0 would make the other
+    // rows' sums NaN, and added for the rows that do attend it at the end
+    __shared__ uint32_t v_special;
+    uint16_t *const kls = fl_smem, *const vls = fl_smem + 2 * C::kBuf;
+    auto swz = [](uint32_t k) { return HD == 128 ? k & 15u : (k >> 1) & 7u; };
+    // the wavefronts' longest contexts, then the splits' statistics: read
+    // before V^T buffer 1 is first written
+    uint32_t *const wmax = reinterpret_cast<uint32_t *>(vls + C::kBuf);
+    const uint32_t tid = threadIdx.x, lane = tid & 63, h = lane >> 5;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t pg = wave % C::kPairGroups, split = wave / C::kPairGroups;
+    // this wavefront's keys of a trip: LDS block and first 32-key tile in it
+    const uint32_t kblk = KS == 4 ? split / 2 : split, t0 = KS == 4 ? split % 2 : 0;
     const uint32_t kvh = blockIdx.x, sq = blockIdx.y, r0 = (gridDim.z - 1 - blockIdx.z) * QT, h0 = kvh * G;
     {
         const uint64_t rows0 = static_cast<uint64_t>(sq) * rows;  // the sequence's first row
-        q += rows0 * n_heads * kFlHd;
-        out += rows0 * n_heads * kFlHd;
+        q += rows0 * n_heads * HD;
+        out += rows0 * n_heads * HD;
         positions += rows0;
         k_cache += sq * seq_cache;
         v_cache += sq * seq_cache;
     }
-    const uint16_t *const kc = k_cache + static_cast<uint64_t>(kvh) * max_len * kFlHd;
-    const uint16_t *const vc = v_cache + static_cast<uint64_t>(kvh) * max_len * kFlHd;
+    const uint16_t *const kc = k_cache + static_cast<uint64_t>(kvh) * max_len * HD;
+    const uint16_t *const vc = v_cache + static_cast<uint64_t>(kvh) * max_len * HD;
 
     // this lane's pair: column l % 32 of its wavefront's score tiles
-    const uint32_t p = wave * 32 + (lane & 31);
+    const uint32_t p = pg * 32 + (lane & 31);
     const bool alive = p < LIVE && r0 + p / G < rows;
     const uint32_t prow = alive ? r0 + p / G : 0, phead = h0 + (alive ? p % G : 0);
     const uint32_t pos = alive ? positions[prow] : 0u;
     const uint32_t ctx = alive ? (pos < max_len ? pos + 1 : max_len) : 0u;
+    if (tid == 0) v_special = 0;
     // the block's longest and shortest live contexts: key blocks below the
     // shortest need no mask
     {
@@ -145,11 +179,11 @@ __global__ __launch_bounds__(kFlThreads) void attn_flash_kernel(
         if (lane == 0) wmax[wave] = static_cast<uint32_t>(mx), wmax[kFlWaves + wave] = static_cast<uint32_t>(mn);
     }
     // q of the pair as B fragments: dims 16 s + 8 h .. + 7
-    uint4 qf[8];
+    uint4 qf[QS];
     {
-        const uint16_t *qp = q + (static_cast<uint64_t>(prow) * n_heads + phead) * kFlHd + 8 * h;
+        const uint16_t *qp = q + (static_cast<uint64_t>(prow) * n_heads + phead) * HD + 8 * h;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
+        for (int s = 0; s < QS; ++s) {
             const uint4 v = *reinterpret_cast<const uint4 *>(qp + 16 * s);
             qf[s] = alive ? v : make_uint4(0u, 0u, 0u, 0u);
         }
@@ -162,60 +196,90 @@ __global__ __launch_bounds__(kFlThreads) void attn_flash_kernel(
         kmin = wmax[kFlWaves + w] < kmin ? wmax[kFlWaves + w] : kmin;
     }
     if (kmax == 0) return;  // no live row (uniform over the block)
-    const uint32_t nkb = (kmax + kFlKeys - 1) / kFlKeys;
+    const uint32_t trips = (kmax + C::kKeys - 1) / C::kKeys;
 
-    // K block kb into LDS by DMA: wavefront w brings keys 8 w .. 8 w + 7 as
-    // two 1 KiB pieces (4 keys x 16 slots each); keys past the block's
+    // trip it's keys into LDS by DMA: wavefront w brings kKeys / 8 of them in
+    // 1 KiB instructions (64 / PP keys x PP slots); keys past the block's
     // longest context read key kmax - 1 (valid, never used)
-    const __amdgpu_buffer_rsrc_t rk = fl_rsrc(kc, static_cast<uint64_t>(max_len) * kFlHd * 2);
-    auto stage_k = [&](uint32_t kb, uint32_t buf) {
+    const __amdgpu_buffer_rsrc_t rk = fl_rsrc(kc, static_cast<uint64_t>(max_len) * HD * 2);
+    constexpr uint32_t kPerWave = C::kKeys / kFlWaves, kPerInst = 64 / PP;
+    auto stage_k = [&](uint32_t it, uint32_t buf) {
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-            const uint32_t kl = 8 * wave + 4 * c + (lane >> 4);  // key within the block
-            uint32_t key = kb * kFlKeys + kl;
+        for (uint32_t c = 0; c < kPerWave / kPerInst; ++c) {
+            const uint32_t k0 = wave * kPerWave + c * kPerInst;
+            const uint32_t kl = k0 + lane / PP;  // key within the trip
+            uint32_t key = it * C::kKeys + kl;
             key = key < kmax ? key : kmax - 1;
-            const uint32_t piece = (lane & 15) ^ (kl & 15);
-            const uint32_t off = static_cast<uint32_t>(k_offset(key, 8 * piece, max_len, kFlHd)) * 2;
+            const uint32_t piece = (lane % PP) ^ swz(kl);
+            const uint32_t off = static_cast<uint32_t>(k_offset(key, 8 * piece, max_len, HD)) * 2;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rk, (__attribute__((address_space(3))) void *)(&kls[buf][(8 * wave + 4 * c) * kFlHd]), 16,
+                rk, (__attribute__((address_space(3))) void *)(kls + buf * C::kBuf + k0 * HD), 16,
                 static_cast<int>(off), 0, 0, 0);
         }
     };
-    // V block kb: thread (key pair i = tid % 32, dim piece c = tid / 32)
-    // loads keys 2 i, 2 i + 1 of dims 8 c .. 8 c + 7, then writes dword
-    // (v[2i][d], v[2i+1][d]) of each dim d to V^T
-    auto load_v = [&](uint32_t kb, uint4 (&v)[2]) {
-        const uint32_t i = tid & 31, c = tid >> 5;
+    // trip it's V: item (key pair i, dim piece c) loads keys 2 i, 2 i + 1 of
+    // dims 8 c .. 8 c + 7, then writes dword (v[2i][d], v[2i+1][d]) of each
+    // dim d to V^T
+    constexpr uint32_t kVPairs = C::kKeys / 2, kVItems = kVPairs * PP;
+    constexpr int kVRounds = kVItems > kFlThreads ? kVItems / kFlThreads : 1;
+    auto load_v = [&](uint32_t it, uint4 (&v)[kVRounds][2]) {
 #pragma unroll
-        for (int e = 0; e < 2; ++e) {
-            uint32_t key = kb * kFlKeys + 2 * i + e;
-            key = key < kmax ? key : kmax - 1;
-            v[e] = *reinterpret_cast<const uint4 *>(vc + static_cast<uint64_t>(key) * kFlHd + 8 * c);
+        for (int r = 0; r < kVRounds; ++r) {
+            const uint32_t item = (tid + r * kFlThreads) % kVItems, i = item % kVPairs, c = item / kVPairs;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                uint32_t key = it * C::kKeys + 2 * i + e;
+                key = key < kmax ? key : kmax - 1;
+                v[r][e] = *reinterpret_cast<const uint4 *>(vc + static_cast<uint64_t>(key) * HD + 8 * c);
+            }
         }
     };
-    auto store_v = [&](const uint4 (&v)[2], uint32_t buf) {
-        const uint32_t i = tid & 31, c = tid >> 5;
-        const uint32_t slot = fl_slot(2 * i);  // even; key 2 i + 1 is the next slot
-        const uint32_t a[4] = {v[0].x, v[0].y, v[0].z, v[0].w}, b[4] = {v[1].x, v[1].y, v[1].z, v[1].w};
+    auto specials = [](uint32_t x) {  // bit 15 / 31: that half is inf or NaN
+        return ((x & 0x7FFF7FFFu) + 0x00800080u) & 0x80008000u;
+    };
+    // masked: some row does not attend all of the trip's keys
+    auto store_v = [&](uint4 (&v)[kVRounds][2], uint32_t buf, bool masked) {
+        if (kVItems < kFlThreads && tid >= kVItems) return;
+        if (masked) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const uint32_t d = 8 * c + e;
-            const uint32_t lo = (a[e / 2] >> (16 * (e % 2))) & 0xFFFFu, hi = (b[e / 2] >> (16 * (e % 2))) & 0xFFFFu;
-            const uint32_t at = d * kFlKeys + (((slot >> 3) ^ ((d >> 1) & 7u)) << 3) + (slot & 7u);
-            *reinterpret_cast<uint32_t *>(&vls[buf][at]) = lo | (hi << 16);
+            for (int r = 0; r < kVRounds; ++r) {
+                uint4 &x = v[r][0], &y = v[r][1];
+                if (specials(x.x) | specials(x.y) | specials(x.z) | specials(x.w) | specials(y.x) | specials(y.y) |
+                    specials(y.z) | specials(y.w)) {
+                    v_special = 1;
+                    auto clear = [&](uint32_t &w) { w &= ~((specials(w) >> 15) * 0xFFFFu); };
+                    clear(x.x), clear(x.y), clear(x.z), clear(x.w);
+                    clear(y.x), clear(y.y), clear(y.z), clear(y.w);
+                }
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < kVRounds; ++r) {
+            const uint32_t item = tid + r * kFlThreads, i = item % kVPairs, c = item / kVPairs;
+            uint16_t *const blk = vls + buf * C::kBuf + i / 32 * (kFlKeys * HD);
+            const uint32_t slot = fl_slot(2 * (i % 32));  // even; key 2 i + 1 is the next slot
+            const uint32_t a[4] = {v[r][0].x, v[r][0].y, v[r][0].z, v[r][0].w};
+            const uint32_t b[4] = {v[r][1].x, v[r][1].y, v[r][1].z, v[r][1].w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t d = 8 * c + e;
+                const uint32_t lo = (a[e / 2] >> (16 * (e % 2))) & 0xFFFFu, hi = (b[e / 2] >> (16 * (e % 2))) & 0xFFFFu;
+                const uint32_t at = d * kFlKeys + (((slot >> 3) ^ ((d >> 1) & 7u)) << 3) + (slot & 7u);
+                *reinterpret_cast<uint32_t *>(blk + at) = lo | (hi << 16);
+            }
         }
     };
-    // S^T of 32-key tile t of a staged block: rows = keys 32 t + 8 (r / 4) +
-    // 4 h + r % 4, column = this lane's pair
-    auto scores = [&](uint32_t buf, int t) {
+    // S^T of 32-key tile t of this wavefront's block of a buffer: rows = keys
+    // 32 t + 8 (r / 4) + 4 h + r % 4, column = this lane's pair
+    auto scores = [&](uint32_t buf, uint32_t t) {
         const uint32_t kl = 32 * t + (lane & 31);
-        const uint16_t *kr = &kls[buf][kl * kFlHd];
+        const uint16_t *kr = kls + buf * C::kBuf + (kblk * kFlKeys + kl) * HD;
         fl_f32x16_t d;
 #pragma unroll
         for (int r = 0; r < 16; ++r) d[r] = 0.f;
 #pragma unroll
-        for (int s = 0; s < 8; ++s) {
-            const uint4 a = *reinterpret_cast<const uint4 *>(kr + (((2 * s + h) ^ (kl & 15)) << 3));
+        for (int s = 0; s < QS; ++s) {
+            const uint4 a = *reinterpret_cast<const uint4 *>(kr + (((2 * s + h) ^ swz(kl)) << 3));
             d = fl_mfma(a, qf[s], d);
         }
         return d;
@@ -225,10 +289,10 @@ __global__ __launch_bounds__(kFlThreads) void attn_flash_kernel(
     // past the pair's context (MASK: the block reaches past some live pair's
     // context)
     const FlExp ex{scale, scale * 1.44269504088896341f};
-    auto score_of = [&](const fl_f32x16_t &d, uint32_t kb, int t, int r, auto mask) {
+    auto score_of = [&](const fl_f32x16_t &d, uint32_t it, uint32_t t, int r, auto mask) {
         const float sv = bf(rne(d[r]));
         if constexpr (decltype(mask)::value) {
-            const uint32_t j = kb * kFlKeys + 32 * t + 8 * (r / 4) + 4 * h + (r % 4);
+            const uint32_t j = it * C::kKeys + kblk * kFlKeys + 32 * t + 8 * (r / 4) + 4 * h + (r % 4);
             return j < ctx ? sv : -INFINITY;
         }
         return sv;
@@ -241,17 +305,18 @@ __global__ __launch_bounds__(kFlThreads) void attn_flash_kernel(
     stage_k(0, 0);
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     __syncthreads();
-    for (uint32_t kb = 0; kb < nkb; ++kb) {
-        const uint32_t buf = kb & 1;
-        if (kb + 1 < nkb) stage_k(kb + 1, buf ^ 1);
+    for (uint32_t it = 0; it < trips; ++it) {
+        const uint32_t buf = it & 1;
+        if (it + 1 < trips) stage_k(it + 1, buf ^ 1);
         auto stats = [&](auto mask) {
 #pragma unroll
-            for (int t = 0; t < 2; ++t) {
+            for (int tt = 0; tt < C::kTiles; ++tt) {
+                const uint32_t t = t0 + tt;
                 const fl_f32x16_t d = scores(buf, t);
                 float sv[16], mt = -INFINITY;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
-                    sv[r] = score_of(d, kb, t, r, mask);
+                    sv[r] = score_of(d, it, t, r, mask);
                     mt = fmaxf(mt, sv[r]);
                 }
                 const float mn = fmaxf(m, mt);
@@ -265,21 +330,39 @@ __global__ __launch_bounds__(kFlThreads) void attn_flash_kernel(
                 }
             }
         };
-        if ((kb + 1) * kFlKeys <= kmin)
+        if ((it + 1) * C::kKeys <= kmin)
             stats(Unmasked{});
         else
             stats(Masked{});
         __builtin_amdgcn_s_waitcnt(0x0f70);  // the next block's DMA has landed
         __syncthreads();
     }
-    // the pair's two halves (lanes l and l ^ 32) combined, the h = 0 half first
+    // two statistics of disjoint keys of a pair, the first one's keys first
+    auto meet = [&](float m0, float l0, float m1, float l1, float *mo, float *lo) {
+        const float mm = fmaxf(m0, m1);
+        const float o = mm == -INFINITY ? 0.f : ex.base(mm);
+        *mo = mm;
+        *lo = (m0 == -INFINITY ? 0.f : l0 * ex(m0, o)) + (m1 == -INFINITY ? 0.f : l1 * ex(m1, o));
+    };
+    // the pair's two halves (lanes l and l ^ 32), the h = 0 half first, then
+    // its splits in order
     float M, S;
     {
         const float mo = __shfl_xor(m, 32, 64), lo = __shfl_xor(l, 32, 64);
-        const float m0 = h ? mo : m, l0 = h ? lo : l, m1 = h ? m : mo, l1 = h ? l : lo;
-        M = fmaxf(m0, m1);
-        const float o = M == -INFINITY ? 0.f : ex.base(M);
-        S = M == -INFINITY ? 1.f : (m0 == -INFINITY ? 0.f : l0 * ex(m0, o)) + (m1 == -INFINITY ? 0.f : l1 * ex(m1, o));
+        meet(h ? mo : m, h ? lo : l, h ? m : mo, h ? l : lo, &M, &S);
+        if constexpr (KS > 1) {
+            float2 *const st = reinterpret_cast<float2 *>(wmax);  // [split][pair]
+            if (h == 0) st[split * C::kPairs + p] = make_float2(M, S);
+            __syncthreads();
+            float2 v = st[p];
+            M = v.x, S = v.y;
+#pragma unroll
+            for (int k = 1; k < KS; ++k) {
+                v = st[k * C::kPairs + p];
+                meet(M, S, v.x, v.y, &M, &S);
+            }
+        }
+        if (M == -INFINITY) S = 1.f;
     }
     // a pair with no key (a dead lane) gets exp(-inf) = 0 everywhere, not NaN
     const float oM = M == -INFINITY ? 0.f : ex.base(M);
@@ -288,34 +371,34 @@ __global__ __launch_bounds__(kFlThreads) void attn_flash_kernel(
 #endif
 
     // Pass 2: p_j = RNE(exp(s_j - M) / S) (masked keys: exp(-inf) = 0), acc +=
-    // P V over 4 tiles of 32 dims
-    fl_f32x16_t acc[4];
+    // P V over DT tiles of 32 dims
+    fl_f32x16_t acc[DT];
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
+    for (int dt = 0; dt < DT; ++dt)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
     {
-        uint4 vr[2];
+        uint4 vr[kVRounds][2];
         stage_k(0, 0);
         load_v(0, vr);
-        store_v(vr, 0);
+        store_v(vr, 0, C::kKeys > kmin);
     }
     __builtin_amdgcn_s_waitcnt(0x0f70);
     __syncthreads();
     fl_f32x16_t dsc;  // the current score tile
-    for (uint32_t kb = 0; kb < nkb; ++kb) {
-        const uint32_t buf = kb & 1;
-        uint4 vr[2];
-        const bool next = kb + 1 < nkb;
+    for (uint32_t it = 0; it < trips; ++it) {
+        const uint32_t buf = it & 1;
+        uint4 vr[kVRounds][2];
+        const bool next = it + 1 < trips;
         if (next) {
-            stage_k(kb + 1, buf ^ 1);
-            load_v(kb + 1, vr);
+            stage_k(it + 1, buf ^ 1);
+            load_v(it + 1, vr);
         }
-        auto probs = [&](int t, uint32_t (&pw)[8], auto mask) {
+        auto probs = [&](uint32_t t, uint32_t (&pw)[8], auto mask) {
 #pragma unroll
             for (int r = 0; r < 16; r += 2) {
                 const fl_f32x16_t &d = dsc;
-                const float s0 = score_of(d, kb, t, r, mask), s1 = score_of(d, kb, t, r + 1, mask);
+                const float s0 = score_of(d, it, t, r, mask), s1 = score_of(d, it, t, r + 1, mask);
 #if FH_FLASH_RCP
                 const float p0 = ex(s0, oM) * rS, p1 = ex(s1, oM) * rS;
 #else
@@ -324,9 +407,10 @@ __global__ __launch_bounds__(kFlThreads) void attn_flash_kernel(
                 pw[r / 2] = f32x2_to_bf16x2_rne(p0, p1);
             }
         };
-        const bool full = (kb + 1) * kFlKeys <= kmin;
+        const bool full = (it + 1) * C::kKeys <= kmin;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
+        for (int tt = 0; tt < C::kTiles; ++tt) {
+            const uint32_t t = t0 + tt;
             dsc = scores(buf, t);
             uint32_t pw[8];  // probabilities as bf16 pairs, in register order
             if (full)
@@ -338,70 +422,154 @@ __global__ __launch_bounds__(kFlThreads) void attn_flash_kernel(
                 const uint4 a = make_uint4(pw[4 * ks], pw[4 * ks + 1], pw[4 * ks + 2], pw[4 * ks + 3]);
                 const uint32_t piece = 2 * (2 * t + ks) + h;  // slots 16 (2 t + ks) + 8 h .. + 7
 #pragma unroll
-                for (int dt = 0; dt < 4; ++dt) {
+                for (int dt = 0; dt < DT; ++dt) {
                     const uint32_t dd = 32 * dt + (lane & 31);
                     const uint4 b = *reinterpret_cast<const uint4 *>(
-                        &vls[buf][dd * kFlKeys + ((piece ^ ((dd >> 1) & 7u)) << 3)]);
+                        vls + buf * C::kBuf + kblk * (kFlKeys * HD) + dd * kFlKeys +
+                        ((piece ^ ((dd >> 1) & 7u)) << 3));
                     acc[dt] = fl_mfma(a, b, acc[dt]);
                 }
             }
         }
-        if (next) store_v(vr, buf ^ 1);  // buffer buf ^ 1 was last read before the previous barrier
+        if (next) store_v(vr, buf ^ 1, (it + 2) * C::kKeys > kmin);  // buffer buf ^ 1 was last read before the previous barrier
         __builtin_amdgcn_s_waitcnt(0x0f70);
         __syncthreads();
     }
 
+    // the splits' sums, in split order (the last trip's barrier is behind)
+    if constexpr (KS > 1) {
+        float *const red = reinterpret_cast<float *>(fl_smem);  // [split - 1][pair group][dt][r][lane]
+        constexpr uint32_t kWaveSums = DT * 16 * 64;
+        if (split > 0) {
+            float *const mine = red + ((split - 1) * C::kPairGroups + pg) * kWaveSums + lane;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) mine[(dt * 16 + r) * 64] = acc[dt][r];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int k = 1; k < KS; ++k) {
+            const float *const part = red + ((k - 1) * C::kPairGroups + pg) * kWaveSums + lane;
+            if (split == 0) {
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[dt][r] += part[(dt * 16 + r) * 64];
+            }
+        }
+    }
+
     // out[row][head][dim]: lane holds dim 32 dt + l % 32 of pairs 8 (r / 4) + 4 h + r % 4
+    if (split == 0) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const uint32_t pp = wave * 32 + 8 * (r / 4) + 4 * h + (r % 4);
-        if (pp >= LIVE || r0 + pp / G >= rows) continue;
-        uint16_t *orow = out + (static_cast<uint64_t>(r0 + pp / G) * n_heads + h0 + pp % G) * kFlHd + (lane & 31);
+        for (int r = 0; r < 16; ++r) {
+            const uint32_t pp = pg * 32 + 8 * (r / 4) + 4 * h + (r % 4);
+            if (pp >= LIVE || r0 + pp / G >= rows) continue;
+            uint16_t *orow = out + (static_cast<uint64_t>(r0 + pp / G) * n_heads + h0 + pp % G) * HD + (lane & 31);
 #pragma unroll
-        for (int dt = 0; dt < 4; ++dt) orow[32 * dt] = rne(acc[dt][r]);
+            for (int dt = 0; dt < DT; ++dt) orow[32 * dt] = rne(acc[dt][r]);
+        }
+    }
+    if (!v_special) return;  // uniform: last written before a barrier of the loop
+
+    // inf and NaN of V in the trips that some row attends in part: p v for
+    // the rows that attend the key, p from the score again
+    __syncthreads();  // the outputs are written, the sums above read
+    float2 *const st = reinterpret_cast<float2 *>(fl_smem);
+    if (split == 0 && h == 0) st[p] = make_float2(oM, S);
+    __syncthreads();
+    for (uint32_t o = tid; o < LIVE * HD; o += kFlThreads) {
+        const uint32_t pp = o / HD, d = o % HD, row = r0 + pp / G;
+        if (row >= rows) continue;
+        const uint64_t at = (static_cast<uint64_t>(row) * n_heads + h0 + pp % G) * HD;
+        const uint32_t rpos = positions[row], rctx = rpos < max_len ? rpos + 1 : max_len;
+        float sum = 0.f;
+        bool any = false;
+        for (uint32_t j = kmin / C::kKeys * C::kKeys; j < rctx; ++j) {
+            const uint32_t v = vc[static_cast<uint64_t>(j) * HD + d];
+            if (!specials(v)) continue;
+            float qk = 0.f;
+            for (uint32_t e = 0; e < HD; ++e) qk = fmaf(bf(q[at + e]), bf(kc[k_offset(j, e, max_len, HD)]), qk);
+            sum += bf(rne(ex(bf(rne(qk)), st[pp].x) / st[pp].y)) * bf(static_cast<uint16_t>(v));
+            any = true;
+        }
+        if (any) out[at + d] = rne(bf(out[at + d]) + sum);
     }
 }
 
-// Whether the one-pass kernel takes `rows` prompt rows of one sequence:
-// head_dim 128, G = n_heads / n_kv of 1 .. 8, and its blocks (n_kv per query
-// tile) fill at least half the CUs.
-bool attention_flash_applies(uint32_t cus, uint32_t rows, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim) {
-    if (head_dim != kFlHd || n_kv == 0 || n_heads % n_kv != 0) return false;
+// Over how many wavefronts the one-pass kernel splits the keys for `batch`
+// sequences of `rows` prompt rows (0: it does not take them): head_dim 64 or
+// 128, G = n_heads / n_kv of 1 .. 8, and query tiles for half the CUs or a
+// prompt of at least 16 rows that is not short against the cache, since a
+// block walks all of its rows' keys (from 1/11 of it, 1/16 for heads of 64).
+// Measured against the two-kernel path, 8 KV heads, 3 query heads each of
+// 128: 100 rows after 1000 keys 32.4 / 35.4 us, 48 after 500 21.4 / 20.4, 48
+// after 2000 50.1 / 37.2, 512 alone 20.1 / 36.5; heads of 64: 24 after 300
+// 10.9 / 14.9, 2048 after 1024 108 / 603.8. The maximum is taken before the
+// scale, which has to be positive, and contexts are compared as floats and
+// keys addressed by 32-bit byte offsets: caches below 2^24 keys.
+// No split where the batch's blocks make two rounds of CUs (8 x 2048 rows, two
+// layers' prompt 14.22 ms against 14.53 over 2 and 15.35 over 4); else over 2
+// where that gives more than a block per CU, 4 otherwise: one 2048-row prompt
+// (256 blocks unsplit, which wait for the one with the most keys) 130.5, 99.4
+// and 135.4 us over 1, 2 and 4, 512 rows 34.8, 23.5 and 19.3.
+uint32_t attention_flash_splits(uint32_t cus, uint32_t batch, uint32_t rows, uint32_t n_heads, uint32_t n_kv,
+                                uint32_t head_dim, uint32_t max_len, float scale) {
+    if (!(scale > 0.f && scale * 1.5f < INFINITY) || max_len >= 1u << 24) return 0;
+    if ((head_dim != 64 && head_dim != 128) || n_kv == 0 || n_heads % n_kv != 0) return 0;
     const uint32_t g = n_heads / n_kv;
-    if (g < 1 || g > 8) return false;
-    const uint64_t tiles = (rows + 256 / g - 1) / (256 / g);
-    return tiles * n_kv * 2 >= cus && tiles <= 65535;
+    if (g < 1 || g > 8) return 0;
+    auto blocks = [&](uint32_t ks) {  // of one sequence
+        const uint32_t qt = 256 / ks / g;
+        return (static_cast<uint64_t>(rows) + qt - 1) / qt * n_kv;
+    };
+    if (2 * blocks(1) < cus && (rows < 16 || max_len > static_cast<uint64_t>(head_dim == 64 ? 16 : 11) * rows)) return 0;
+    const uint32_t ks = blocks(1) * batch >= 2ull * cus ? 1 : blocks(2) > cus ? 2 : 4;
+    return blocks(ks) / n_kv > 65535 ? 0 : ks;
+}
+
+template <int HD, int G, int KS>
+static void launch_flash(hipStream_t stream, const uint16_t *q, const uint32_t *positions, uint32_t rows,
+                         const uint16_t *k_cache, const uint16_t *v_cache, uint32_t n_heads, uint32_t n_kv,
+                         uint32_t max_len, float scale, uint16_t *out, uint32_t batch, uint64_t seq_cache) {
+    using C = FlCfg<HD, KS>;
+    static const hipError_t opt_in =
+        hipFuncSetAttribute(reinterpret_cast<const void *>(attn_flash_kernel<HD, G, KS>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds);
+    (void)opt_in;
+    constexpr uint32_t QT = C::kPairs / G;
+    hipLaunchKernelGGL((attn_flash_kernel<HD, G, KS>), dim3(n_kv, batch, (rows + QT - 1) / QT), dim3(kFlThreads),
+                       C::kLds, stream, q, positions, rows, k_cache, v_cache, seq_cache, n_heads, max_len, scale, out);
 }
 
 // Launches the one-pass kernel over `batch` sequences of `rows` rows (q, out
 // and positions consecutive per sequence, caches seq_cache elements apart)
-// when attention_flash_applies to one sequence; returns false otherwise (the
-// caller takes the two-kernel path). Every block is the one a launch per
-// sequence would run, so the outputs are those of per-sequence launches.
+// when attention_flash_splits takes them; returns false otherwise (the caller
+// takes the two-kernel path). Where one sequence alone splits its keys alike,
+// every block is the one a launch per sequence would run.
 bool launch_attention_flash(hipStream_t stream, uint32_t cus, const uint16_t *q, const uint32_t *positions,
                             uint32_t rows, const uint16_t *k_cache, const uint16_t *v_cache, uint32_t n_heads,
                             uint32_t n_kv, uint32_t head_dim, uint32_t max_len, float scale, uint16_t *out,
                             uint32_t batch, uint64_t seq_cache) {
-    if (batch == 0 || batch > 65535 || !attention_flash_applies(cus, rows, n_heads, n_kv, head_dim)) return false;
+    const uint32_t ks = attention_flash_splits(cus, batch, rows, n_heads, n_kv, head_dim, max_len, scale);
+    if (batch == 0 || batch > 65535 || ks == 0) return false;
     const uint32_t g = n_heads / n_kv;
-    const uint32_t tiles = (rows + 256 / g - 1) / (256 / g);
-    const dim3 grid(n_kv, batch, tiles);
-#define FH_FLASH_G(GG)                                                                                          \
-    case GG:                                                                                                    \
-        hipLaunchKernelGGL(attn_flash_kernel<GG>, grid, dim3(kFlThreads), 0, stream, q, positions, rows, k_cache, \
-                           v_cache, seq_cache, n_heads, max_len, scale, out);                                   \
-        return true;
-    switch (g) {
-        FH_FLASH_G(1)
-        FH_FLASH_G(2)
-        FH_FLASH_G(3)
-        FH_FLASH_G(4)
-        FH_FLASH_G(5)
-        FH_FLASH_G(6)
-        FH_FLASH_G(7)
-        FH_FLASH_G(8)
+#define FH_FLASH(HH, GG, SS)                                                                                  \
+    if (head_dim == HH && g == GG && ks == SS) {                                                              \
+        launch_flash<HH, GG, SS>(stream, q, positions, rows, k_cache, v_cache, n_heads, n_kv, max_len, scale, \
+                                 out, batch, seq_cache);                                                      \
+        return true;                                                                                          \
     }
+#define FH_FLASH_KS(HH, GG) FH_FLASH(HH, GG, 1) FH_FLASH(HH, GG, 2) FH_FLASH(HH, GG, 4)
+#define FH_FLASH_G(HH)                                                                        \
+    FH_FLASH_KS(HH, 1) FH_FLASH_KS(HH, 2) FH_FLASH_KS(HH, 3) FH_FLASH_KS(HH, 4) FH_FLASH_KS(HH, 5) \
+    FH_FLASH_KS(HH, 6) FH_FLASH_KS(HH, 7) FH_FLASH_KS(HH, 8)
+    FH_FLASH_G(64)
+    FH_FLASH_G(128)
 #undef FH_FLASH_G
+#undef FH_FLASH_KS
+#undef FH_FLASH
     return false;
 }
 

@@ -153,7 +153,7 @@ def assert_attention_close(got, ref, flip, what):
     assert ok.all(), (what, np.argwhere(~ok)[:4].tolist(), int(u.max()))
 
 
-def run_attention(device, q, kc, vc, pos, ws=None):
+def run_attention(device, q, kc, vc, pos, ws=None, scale=None):
     t, n_heads, hd = q.shape
     n_kv, max_len, _ = kc.shape
     s = [up(device, a) for a in (q, tile_k(kc), vc, np.ascontiguousarray(pos, dtype=np.uint32))]
@@ -161,7 +161,8 @@ def run_attention(device, q, kc, vc, pos, ws=None):
     if ws is None:
         ws = device.zeros(nbytes)
     out = device.empty(t * n_heads * hd * 2)
-    scale = float(np.float32(1) / np.sqrt(np.float32(hd), dtype=np.float32))
+    if scale is None:
+        scale = float(np.float32(1) / np.sqrt(np.float32(hd), dtype=np.float32))
     _lib.call("fh_attention", device.handle, ctypes.c_void_p(s[0].ptr), ctypes.c_void_p(s[1].ptr),
               ctypes.c_void_p(s[2].ptr), ctypes.c_void_p(s[3].ptr), t, n_heads, n_kv, hd, max_len,
               ctypes.c_float(scale), ctypes.c_void_p(ws.ptr), nbytes, ctypes.c_void_p(out.ptr))
@@ -220,6 +221,80 @@ def test_attention_one_pass_prefill(device, n_heads, n_kv, t, max_len, past):
     assert_attention_close(got[rows], ref[rows], flip[rows], rows)
     again, _, _ = run_attention(device, q, kc, vc, pos)
     assert np.array_equal(got, again), "one-pass attention differs between runs"
+
+
+# The one-pass kernel's key splits: 4 (few query tiles: ragged last tiles, one
+# trip of keys, a context that ends inside a wavefront's run of keys, groups of
+# 7 and 8 heads), 2 (a block per CU) and none (two rounds), head sizes 64 and
+# 128, and prompts too short against their cache, which the two-kernel path
+# keeps. One position lies past the cache (it attends all of it).
+FLASH_SPLIT_CASES = [(32, 8, 64, 40, 100, 50), (32, 8, 64, 700, 901, 201), (32, 8, 64, 1100, 1190, 90),
+                     (64, 64, 64, 2048, 2060, 12), (4, 2, 128, 16, 16, 0), (24, 8, 128, 100, 161, 61),
+                     (14, 2, 128, 130, 1030, 900), (16, 2, 128, 65, 97, 32), (32, 8, 128, 1024, 1088, 64),
+                     (24, 8, 128, 24, 300, 276), (32, 8, 64, 16, 257, 241)]
+
+
+@pytest.mark.parametrize("n_heads,n_kv,hd,t,max_len,past", FLASH_SPLIT_CASES)
+def test_attention_one_pass_key_splits(device, n_heads, n_kv, hd, t, max_len, past):
+    q = synth.bf16_normal(31, (t, n_heads, hd))
+    kc = synth.bf16_normal(32, (n_kv, max_len, hd))
+    vc = synth.bf16_normal(33, (n_kv, max_len, hd))
+    pos = (past + np.arange(t)).astype(np.uint32)
+    pos[t // 2] = max_len + 5
+    got, scale, _ = run_attention(device, q, kc, vc, pos)
+    rng = np.random.default_rng(t + max_len)
+    rows = sorted(set([0, 1, t // 2, t - 2, t - 1] + rng.integers(0, t, 6).tolist()))
+    ref, flip = attention_ref(q, kc, vc, pos, scale, rows)
+    assert_attention_close(got[rows], ref[rows], flip[rows], rows)
+    again, _, _ = run_attention(device, q, kc, vc, pos)
+    assert np.array_equal(got, again), "one-pass attention differs between runs"
+
+
+# inf and NaN of V reach only the rows that attend their keys, and only in
+# their dim (KS 4, 2 and none; positions out of order, so that many trips hold
+# keys that only some rows attend)
+@pytest.mark.parametrize("n_heads,n_kv,hd,t,past", [(32, 8, 64, 70, 30), (8, 2, 128, 200, 0), (32, 8, 64, 1100, 0),
+                                                    (64, 64, 64, 2048, 0)])
+def test_attention_one_pass_special_values(device, n_heads, n_kv, hd, t, past):
+    max_len = past + t
+    q = synth.bf16_normal(41, (t, n_heads, hd))
+    kc = synth.bf16_normal(42, (n_kv, max_len, hd))
+    vc = synth.bf16_normal(43, (n_kv, max_len, hd))
+    pos = past + np.arange(t)
+    pos[t // 3], pos[t // 2] = past, max_len + 9
+    ctx = np.minimum(pos, max_len - 1) + 1
+    g = n_heads // n_kv
+    spots = [(0, past + t // 2, 5, 0x7F80), (n_kv - 1, max_len - 1, hd - 1, 0x7FC0), (0, past + 2, 0, 0xFF80),
+             (1, past + t // 2 + 1, 6, 0xFF80)]
+    for kv, j, d, _ in spots:
+        vc[kv, j, d] = 0
+    clean, _, _ = run_attention(device, q, kc, vc, pos)
+    for kv, j, d, value in spots:
+        vc[kv, j, d] = value
+    got, _, _ = run_attention(device, q, kc, vc, pos)
+    hit = np.zeros(got.shape, dtype=bool)
+    for kv, j, d, value in spots:
+        rows = np.nonzero(ctx > j)[0]
+        hit[rows, kv * g:(kv + 1) * g, d] = True
+        vals = R.from_bf16(got[rows][:, kv * g:(kv + 1) * g, d])
+        assert not np.isfinite(vals).any()
+        assert (np.isnan(vals) | (vals == R.from_bf16(np.array([value], np.uint16)))).all()
+        assert value == 0x7FC0 or (vals == R.from_bf16(np.array([value], np.uint16))).any()
+    assert np.array_equal(got[~hit], clean[~hit])
+
+
+# scales the one-pass kernel does not take: equal weights at 0, and the lowest
+# scores first below it
+@pytest.mark.parametrize("scale", [0.0, -0.125])
+def test_attention_scale_not_positive(device, scale):
+    t, n_heads, n_kv, hd = 150, 16, 8, 64
+    q = synth.bf16_normal(51, (t, n_heads, hd))
+    kc = synth.bf16_normal(52, (n_kv, t, hd))
+    vc = synth.bf16_normal(53, (n_kv, t, hd))
+    got, _, _ = run_attention(device, q, kc, vc, np.arange(t), scale=scale)
+    rows = [0, 1, 15, 64, 149]
+    ref, flip = attention_ref(q, kc, vc, np.arange(t), scale, rows)
+    assert_attention_close(got[rows], ref[rows], flip[rows], rows)
 
 
 def test_attention_workspace_reuse(device):
