@@ -129,6 +129,7 @@ SIGNATURES = {
     "fh_synchronize": [_vp],
     "fh_device_stream": [_vp, ctypes.POINTER(_vp)],
     "fh_alloc": [_vp, _sz, _int, ctypes.POINTER(_vp)],
+    "fh_alloc_output": [_vp, _sz, ctypes.POINTER(_vp)],
     "fh_free": [_vp, _vp],
     "fh_upload": [_vp, _vp, _vp, _sz],
     "fh_download": [_vp, _vp, _vp, _sz],

@@ -392,8 +392,11 @@ int fh_device_stream(fh_device *dev, void **stream) {
     return FH_OK;
 }
 
-int fh_alloc(fh_device *dev, size_t nbytes, int zero_fill, void **out) {
-    const char *fn = "fh_alloc";
+// fh_alloc and fh_alloc_output. Work queued on the stream may still use a kept
+// block: unless `ordered` says that an op on that stream writes it first (or
+// the clearing below does), the caller may touch it from anywhere, so the
+// work is waited for, as fh_free did before it kept blocks.
+static int allocate(fh_device *dev, size_t nbytes, int zero_fill, bool ordered, void **out, const char *fn) {
     if (!out) return fail(FH_ERR_INVALID_ARGUMENT, "%s: out is null", fn);
     *out = nullptr;
     if (int rc = check_usable(dev, fn)) return rc;
@@ -402,6 +405,14 @@ int fh_alloc(fh_device *dev, size_t nbytes, int zero_fill, void **out) {
     const size_t size = std::max<size_t>(nbytes, 1);
     void *p = take_pooled(dev, size);
     hipError_t err = hipSuccess;
+    if (p != nullptr && !ordered && !zero_fill) {
+        err = hipStreamSynchronize(dev->stream);
+        if (err != hipSuccess) {
+            hipFree(p);
+            dev->capacity.erase(reinterpret_cast<uintptr_t>(p));
+            return device_error(dev, err, fn, "hipStreamSynchronize");
+        }
+    }
     if (p == nullptr) {
         err = hipMalloc(&p, size);
         if ((err != hipSuccess || p == nullptr) && !dev->pool.empty()) {
@@ -430,6 +441,14 @@ int fh_alloc(fh_device *dev, size_t nbytes, int zero_fill, void **out) {
     note_allocation(dev, size);
     *out = p;
     return FH_OK;
+}
+
+int fh_alloc(fh_device *dev, size_t nbytes, int zero_fill, void **out) {
+    return allocate(dev, nbytes, zero_fill, false, out, "fh_alloc");
+}
+
+int fh_alloc_output(fh_device *dev, size_t nbytes, void **out) {
+    return allocate(dev, nbytes, 0, true, out, "fh_alloc_output");
 }
 
 int fh_free(fh_device *dev, void *ptr) {

@@ -224,8 +224,14 @@ class HipDevice:
         return self._alloc(nbytes, zero=True)
 
     def empty(self, nbytes: int) -> HipStorage:
-        """Uninitialised storage (an op's output)."""
+        """Uninitialised storage."""
         return self._alloc(nbytes, zero=False)
+
+    def _output(self, nbytes: int) -> HipStorage:
+        """Uninitialised storage that an op on the stream writes first."""
+        ptr = ctypes.c_void_p()
+        _lib.call("fh_alloc_output", self.handle, nbytes, ctypes.byref(ptr))
+        return HipStorage(self, ptr.value, nbytes)
 
     def storage_to_bytes(self, operand: Operand) -> bytes:
         if not operand.layout.is_contiguous():
@@ -251,7 +257,7 @@ class HipDevice:
         numel = 1
         for d in shape:
             numel *= d
-        out = self.empty(numel * out_dtype.itemsize)
+        out = self._output(numel * out_dtype.itemsize)
         if isinstance(op, QuantizedMatmul):
             x, wq, s, b = inputs
             for w in (wq, s, b):
@@ -266,7 +272,7 @@ class HipDevice:
                 # src/metal/mod.rs:384-401): rows the kernel cannot read in
                 # place (a column stride, overlapping or broadcast rows) are
                 # copied to a contiguous [rows, k] first.
-                staged = self.empty(rows * k * 2)
+                staged = self._output(rows * k * 2)
                 _lib.call("fh_copy_strided", self.handle, int(x.dtype), ctypes.c_void_p(x.storage.ptr),
                           ctypes.byref(x.layout.view()), ctypes.c_void_p(staged.ptr))
                 x_ptr, x_ld = staged.ptr, k

@@ -109,6 +109,10 @@ int fh_device_stream(fh_device *dev, void **stream);
  * zero_fill != 0 the memory is cleared before any later op on the stream
  * reads it (Device::zeros). */
 int fh_alloc(fh_device *dev, size_t nbytes, int zero_fill, void **out);
+/* The same without the clearing, for storage that an op on the device's
+ * stream writes before anything else touches it (an op's output): a block
+ * kept by fh_free is handed out without a wait for the work queued on it. */
+int fh_alloc_output(fh_device *dev, size_t nbytes, void **out);
 /* Frees an allocation of this device. Work already queued on the device's
  * stream may still use the memory; it is then kept for later fh_alloc calls
  * of the device (at most 512 MiB, blocks of at most 128 MiB, the oldest given

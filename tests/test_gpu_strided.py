@@ -550,3 +550,35 @@ def test_freed_blocks_are_reused_in_stream_order(nbytes):
         assert dev.run_memory_peak()["bytes"] == base
     finally:
         dev.close()
+
+
+@pytest.mark.parametrize("kept", [True, False])
+def test_fresh_storage_is_idle_on_return(kept):
+    """Storage from empty() may be written from any stream at once: the queued
+    work that still uses a kept block has ended by then. Op outputs are not
+    waited for (the op writes them in stream order) and hold the op's result."""
+    dev = HipDevice(0)
+    try:
+        ptr = ctypes.c_void_p()
+        _lib.call("fh_device_stream", dev.handle, ctypes.byref(ptr))
+        query = _lib.load().hipStreamQuery  # found through the library's own dependency
+        query.argtypes = [ctypes.c_void_p]
+        n = 1024
+        an = np.random.default_rng(7).standard_normal((n, n)).astype(np.float32)
+        a = f32(dev, an, an.shape)
+        dev.synchronize()
+        out = None
+        for _ in range(40):
+            out = a.matmul(dev, a)
+        want = out.to_numpy(dev)
+        for _ in range(40):
+            out = a.matmul(dev, a)
+        nbytes = n * n * 4
+        del out  # its kernel is still queued
+        fresh = dev.empty(nbytes if kept else 2 * nbytes)
+        if kept:
+            assert query(ptr) == 0
+        del fresh
+        assert np.array_equal(a.matmul(dev, a).to_numpy(dev), want)
+    finally:
+        dev.close()
