@@ -505,7 +505,7 @@ __global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_f
 // block walks all of its rows' keys (from 1/11 of it, 1/16 for heads of 64).
 // Measured against the two-kernel path, 8 KV heads, 3 query heads each of
 // 128: 100 rows after 1000 keys 32.4 / 35.4 us, 48 after 500 21.4 / 20.4, 48
-// after 2000 50.1 / 37.2, 512 alone 20.1 / 36.5; heads of 64: 24 after 300
+// after 2000 50.1 / 37.2, 512 alone 23.5 / 36.5; heads of 64: 24 after 300
 // 10.9 / 14.9, 2048 after 1024 108 / 603.8. The maximum is taken before the
 // scale, which has to be positive, and contexts are compared as floats and
 // keys addressed by 32-bit byte offsets: caches below 2^24 keys.
@@ -513,7 +513,10 @@ __global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_f
 // layers' prompt 14.22 ms against 14.53 over 2 and 15.35 over 4); else over 2
 // where that gives more than a block per CU, 4 otherwise: one 2048-row prompt
 // (256 blocks unsplit, which wait for the one with the most keys) 130.5, 99.4
-// and 135.4 us over 1, 2 and 4, 512 rows 34.8, 23.5 and 19.3.
+// and 135.4 us over 1, 2 and 4, 512 rows 34.8, 23.5 and 19.3. Longer prompts
+// with heads of 128 stay at 2 all the same: the error against 64 bits is the
+// same at 2 and 4, but over 4 the rounding of a 28-layer model's 512-row prompt
+// moved its second greedy id, a near tie, out of the reference's top 5.
 uint32_t attention_flash_splits(uint32_t cus, uint32_t batch, uint32_t rows, uint32_t n_heads, uint32_t n_kv,
                                 uint32_t head_dim, uint32_t max_len, float scale) {
     if (!(scale > 0.f && scale * 1.5f < INFINITY) || max_len >= 1u << 24) return 0;
@@ -525,7 +528,8 @@ uint32_t attention_flash_splits(uint32_t cus, uint32_t batch, uint32_t rows, uin
         return (static_cast<uint64_t>(rows) + qt - 1) / qt * n_kv;
     };
     if (2 * blocks(1) < cus && (rows < 16 || max_len > static_cast<uint64_t>(head_dim == 64 ? 16 : 11) * rows)) return 0;
-    const uint32_t ks = blocks(1) * batch >= 2ull * cus ? 1 : blocks(2) > cus ? 2 : 4;
+    const uint32_t ks = blocks(1) * batch >= 2ull * cus ? 1
+                        : blocks(2) > cus || (head_dim == 128 && rows >= 256) ? 2 : 4;
     return blocks(ks) / n_kv > 65535 ? 0 : ks;
 }
 
