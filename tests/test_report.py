@@ -8,6 +8,7 @@ import os
 import numpy as np
 import pytest
 
+from foundry_amd import _lib, report
 from foundry_amd.report import BenchConfig, BenchError, draw_inputs, git_commit, metrics_from_runs, percentile, summary
 
 GOLDEN = os.path.join(os.path.dirname(__file__), "golden", "prompt_ids_seed0_vocab128256.json")
@@ -123,3 +124,13 @@ def test_draw_inputs_order_and_golden_prompt():
     assert np.array_equal(flat, draw_inputs(BenchConfig(prompt_token_count=16, batch_size=1), 128256)[1][0])
     _, _, s3 = draw_inputs(BenchConfig(prompt_token_count=0, new_token_count=3, batch_size=2), 128256)
     assert s3.shape == (2,)
+
+
+@pytest.mark.parametrize("name", ["fh_alloc", "fh_alloc_output", "fh_free"])
+def test_call_timer_counts_no_allocation(monkeypatch, name):
+    """Allocating and freeing storage are no dispatches of a step's profile."""
+    seen = []
+    monkeypatch.setattr(_lib, "call", lambda n, *args: seen.append(n))
+    with report._CallTimer(None) as timer:  # a timed call would need the device
+        _lib.call(name, 1, 2)
+    assert seen == [name] and timer.kernels == {}
