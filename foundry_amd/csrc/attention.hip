@@ -34,10 +34,11 @@
 //       rows.
 //   fh_attention with head_dim 128 uses attn_pv_tile_kernel instead: the
 //   query-row tiles of the scores, P.V on the matrix cores (M and S combined
-//   over each row's chunks in another fixed order). A prompt that is not
-//   short against its cache takes one launch of attn_flash_kernel instead
-//   (attention_flash.hip, attention_flash_splits): both passes over the keys
-//   in one block per tile, no workspace.
+//   over each row's chunks in another fixed order). A prompt whose 256-pair
+//   query tiles fill half the device, or with heads of 64 one that is not
+//   short against its cache, takes one launch of attn_flash_kernel instead
+//   (attention_flash.hip, flash_plan): both passes over the keys in one block
+//   per tile, no workspace.
 //   Every output element is a sum in a fixed order, so results do not
 //   change from run to run.
 // splits and slices make rows * n_kv * (blocks per pair) about
@@ -766,6 +767,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_chunk_kernel(
 // (8 keys of one dim) is one 16-byte read. The wavefronts' sums are added in
 // order through LDS: one chunk writes RNE(out), several write f32 partials
 // for attn_combine_kernel. Rows with no key in the chunk write nothing.
+// An inf or NaN of V whose key not every row of the tile attends is staged as
+// 0, since its probability of 0 would make the other rows' sums NaN, and added
+// at the end for the rows that do attend it.
 constexpr int kPvtPitch = 40;  // bf16 per transposed V row in LDS: 32 keys + 8 of padding
 
 template <int HD, int G>
@@ -780,17 +784,20 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
     static_assert(sizeof(uint16_t) * kAttnWaves * HD * kPvtPitch >= sizeof(float) * kAttnWaves * 16 * HD,
                   "the wavefronts' sums fit the transposed-V area");
     __shared__ __align__(16) uint16_t vt[kAttnWaves][HD][kPvtPitch];
+    __shared__ uint32_t special[kAttnWaves];  // a wavefront staged an inf or NaN as 0
+    __shared__ float2 row_ms[16];
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 15, quad = lane >> 4;
     const uint32_t kvh = blockIdx.x / chunks, c = blockIdx.x % chunks;
     const uint32_t r0 = blockIdx.y * R, h0 = kvh * G;
     uint32_t ctxq[R];
-    uint32_t cmax = 0;
+    uint32_t cmax = 0, cmin = max_len;
 #pragma unroll
     for (uint32_t qi = 0; qi < R; ++qi) {
         const uint32_t r = r0 + qi;
         const uint32_t p = r < rows ? positions[r] : 0u;
         ctxq[qi] = r < rows ? (p < max_len ? p + 1 : max_len) : 0u;
         cmax = ctxq[qi] > cmax ? ctxq[qi] : cmax;
+        if (r < rows) cmin = ctxq[qi] < cmin ? ctxq[qi] : cmin;
     }
     const uint32_t k0 = c * chunk_keys;
     const uint32_t kend = k0 + chunk_keys < cmax ? k0 + chunk_keys : cmax;  // keys the tile reads in this chunk
@@ -845,6 +852,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
     uint16_t(*vw)[kPvtPitch] = vt[wave];
     uint4 va[8];
     float sa[8];
+    bool cleared = false;
     uint32_t s = wave;
     if (s < nsteps) {
         load_v(s, va);
@@ -857,6 +865,10 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
         if (more) {  // the next step's loads are in flight while this one is used
             load_v(s + kAttnWaves, vn);
             load_s(s + kAttnWaves, sn);
+        }
+        if (k0 + s * 32 + 32 > cmin) {  // some row does not attend all of the step's keys
+#pragma unroll
+            for (int t = 0; t < 8; ++t) cleared |= clear_specials(va[t]);
         }
         // transpose: dim 8 pv + d of keys 8 vj .. 8 vj + 7 as one 16-byte row piece
 #pragma unroll
@@ -895,6 +907,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
             for (int e = 0; e < 8; ++e) sa[e] = sn[e];
         }
     }
+    const uint32_t wave_cleared = __any(cleared) ? 1u : 0u;
+    if (lane == 0) special[wave] = wave_cleared;
+    if (wave == 0 && quad == 0) row_ms[col] = make_float2(mrow, srow_sum);
     // the wavefronts' sums, added in wavefront order: result lane (dim col of
     // tile t, row quad) holds rows 4 quad + i
     __syncthreads();  // every wavefront is done with its V slice
@@ -904,6 +919,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
 #pragma unroll
         for (int i = 0; i < 4; ++i) red[wave][quad * 4 + i][16 * t + col] = acc[t][i];
     __syncthreads();
+    uint32_t any_special = 0;
+#pragma unroll
+    for (int w = 0; w < kAttnWaves; ++w) any_special |= special[w];
     for (uint32_t o = tid; o < LIVE * HD; o += kAttnThreads) {
         const uint32_t rr = o / HD, d = o % HD, qi = rr / G, h = rr % G;
         uint32_t ctx_r = 0;
@@ -911,8 +929,18 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
         for (uint32_t q = 0; q < R; ++q)
             if (q == qi) ctx_r = ctxq[q];
         if (k0 >= ctx_r) continue;  // past the row's context, or a row past the last
-        const float v = ((red[0][rr][d] + red[1][rr][d]) + red[2][rr][d]) + red[3][rr][d];
+        float v = ((red[0][rr][d] + red[1][rr][d]) + red[2][rr][d]) + red[3][rr][d];
         const uint32_t r = r0 + qi;
+        if (any_special) {  // keys of the steps that were staged so, k0 + 32 ((cmin - k0) / 32) on
+            const uint16_t *const sr = scores + (static_cast<uint64_t>(r) * n_heads + h0 + h) * max_len;
+            const uint16_t *const vd = v_cache + static_cast<uint64_t>(kvh) * max_len * HD + d;
+            const uint32_t end = ctx_r < kend ? ctx_r : kend;
+            for (uint32_t j = cmin > k0 ? cmin - (cmin - k0) % 32 : k0; j < end; ++j) {
+                const uint16_t x = vd[static_cast<uint64_t>(j) * HD];
+                if (!bf16_specials(x)) continue;
+                v += bf(rne(expf(score_of(sr[j], scale) - row_ms[rr].x) / row_ms[rr].y)) * bf(x);
+            }
+        }
         if (chunks == 1)
             out[(static_cast<uint64_t>(r) * n_heads + h0 + h) * HD + d] = rne(v);
         else

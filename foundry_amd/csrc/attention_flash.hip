@@ -8,9 +8,9 @@
 //
 // Design for CDNA4: block (KV head, tile of 256 / G query rows), 8 wavefronts;
 // the tile's (row, head) pairs are the columns of the score tiles, 32 per
-// wavefront. (With few tiles the keys are split over 2 or 4 wavefronts
-// instead, and a block holds 128 or 64 pairs.) The keys are walked twice, 64
-// or 128 at a time through LDS:
+// wavefront. (With few tiles, heads of 128 take blocks of 4 wavefronts, and
+// heads of 64 split their keys over 2 or 4 wavefronts; a block then holds 128
+// or 64 pairs.) The keys are walked twice, 64 or 128 at a time through LDS:
 //   pass 1: S^T = K Q^T on the matrix cores (v_mfma_f32_32x32x16_bf16, the
 //     keys as A rows, the pairs' q as B columns held in registers for the
 //     whole block), so a lane holds 16 keys of ONE pair: the running max and
@@ -34,16 +34,16 @@ namespace fh {
 
 namespace {
 
-constexpr int kFlThreads = 512;
-constexpr int kFlWaves = kFlThreads / 64;
 constexpr int kFlKeys = 64;  // keys per LDS block
 
-// Shape of a block: head size, and over how many wavefronts KS the keys of a
-// (row, head) pair are split (1, 2 or 4; the block then holds 256 / KS pairs).
-template <int HD, int KS>
+// Shape of a block: head size, wavefronts W, and over how many of them KS the
+// keys of a (row, head) pair are split (1, 2 or 4).
+template <int HD, int W, int KS>
 struct FlCfg {
-    static constexpr int kPairGroups = kFlWaves / KS;      // wavefronts of 32 pairs each
-    static constexpr uint32_t kPairs = 32 * kPairGroups;
+    static constexpr int kThreads = 64 * W;
+    static constexpr int kPairGroups = W / KS;             // wavefronts of 32 pairs each
+    static constexpr uint32_t kPairs = 32 * kPairGroups;   // of the block
+    static constexpr uint32_t kParts = 8 / W;              // blocks that share a query tile
     static constexpr int kBlocks = KS == 1 ? 1 : 2;        // LDS blocks of 64 keys per trip
     static constexpr uint32_t kKeys = kFlKeys * kBlocks;   // keys per trip
     static constexpr int kTiles = KS == 4 ? 1 : 2;         // 32-key tiles a wavefront takes of them
@@ -117,19 +117,24 @@ struct FlExp {
 // [max_len][HD]) over its cache. positions[r]: the row's position; it attends
 // keys 0 .. min(pos, max_len - 1). Tiles go out last first: a prompt's later
 // rows attend more keys, and the longest blocks then start first.
-// With KS > 1 wavefront w holds pairs 32 (w % (8 / KS)) .. + 31 and every KS-th
+// With W = 4 a block holds half of the pairs of a 256-pair tile. It walks the
+// whole tile's keys, so a pair's sums are those of the block of 8: a running
+// sum is rescaled at every trip, also past the pair's last key, and that can
+// move it by an ulp.
+// With KS > 1 wavefront w holds pairs 32 (w % (W / KS)) .. + 31 and every KS-th
 // run of 64 (KS = 4: 32) keys; the splits' statistics, and at the end their
 // sums of P.V, meet in LDS and are added in split order. Two blocks share a CU
 // where their registers allow it (heads of 64, 128 of them a lane: 2048 rows
 // after 1024 108 us, 124 at 130 registers).
-template <int HD, int G, int KS>
-__global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_flash_kernel(
+template <int HD, int G, int W, int KS>
+__global__ __launch_bounds__(64 * W, HD == 64 && KS > 1 ? 4 : 2) void attn_flash_kernel(
     const uint16_t *__restrict__ q, const uint32_t *__restrict__ positions, uint32_t rows,
     const uint16_t *__restrict__ k_cache, const uint16_t *__restrict__ v_cache, uint64_t seq_cache, uint32_t n_heads,
     uint32_t max_len, float scale, uint16_t *__restrict__ out) {
-    using C = FlCfg<HD, KS>;
-    constexpr uint32_t QT = C::kPairs / G;  // query rows per block
-    constexpr uint32_t LIVE = QT * G;       // (row, head) pairs of the block
+    using C = FlCfg<HD, W, KS>;
+    constexpr uint32_t PARTS = C::kParts;          // blocks per query tile
+    constexpr uint32_t QT = C::kPairs * PARTS / G;  // query rows per tile
+    constexpr uint32_t LIVE = QT * G;               // (row, head) pairs of the tile
     constexpr int QS = HD / 16;             // MFMA k steps of a score
     constexpr int DT = HD / 32;             // 32-dim tiles of the output
     constexpr uint32_t PP = HD / 8;         // 16-byte pieces per key
@@ -152,7 +157,9 @@ __global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_f
     const uint32_t pg = wave % C::kPairGroups, split = wave / C::kPairGroups;
     // this wavefront's keys of a trip: LDS block and first 32-key tile in it
     const uint32_t kblk = KS == 4 ? split / 2 : split, t0 = KS == 4 ? split % 2 : 0;
-    const uint32_t kvh = blockIdx.x, sq = blockIdx.y, r0 = (gridDim.z - 1 - blockIdx.z) * QT, h0 = kvh * G;
+    const uint32_t order = gridDim.z - 1 - blockIdx.z, p0 = order % PARTS * C::kPairs;
+    const uint32_t kvh = blockIdx.x, sq = blockIdx.y, r0 = order / PARTS * QT, h0 = kvh * G;
+    if (r0 + p0 / G >= rows) return;  // no live pair (uniform over the block)
     {
         const uint64_t rows0 = static_cast<uint64_t>(sq) * rows;  // the sequence's first row
         q += rows0 * n_heads * HD;
@@ -165,18 +172,28 @@ __global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_f
     const uint16_t *const vc = v_cache + static_cast<uint64_t>(kvh) * max_len * HD;
 
     // this lane's pair: column l % 32 of its wavefront's score tiles
-    const uint32_t p = pg * 32 + (lane & 31);
+    const uint32_t pb = pg * 32 + (lane & 31), p = p0 + pb;  // in the block, in the tile
     const bool alive = p < LIVE && r0 + p / G < rows;
     const uint32_t prow = alive ? r0 + p / G : 0, phead = h0 + (alive ? p % G : 0);
     const uint32_t pos = alive ? positions[prow] : 0u;
     const uint32_t ctx = alive ? (pos < max_len ? pos + 1 : max_len) : 0u;
     if (tid == 0) v_special = 0;
-    // the block's longest and shortest live contexts: key blocks below the
-    // shortest need no mask
+    // the tile's longest and the block's shortest live contexts: key blocks
+    // below the shortest need no mask
     {
-        const float mx = wave_max(static_cast<float>(ctx));
+        uint32_t most = ctx;
+        if constexpr (PARTS > 1) {  // the other half's pair
+            const uint32_t o = (p + C::kPairs) % (PARTS * C::kPairs);
+            const uint32_t orow = r0 + o / G;
+            if (o < LIVE && orow < rows) {
+                const uint32_t opos = positions[orow];
+                const uint32_t octx = opos < max_len ? opos + 1 : max_len;
+                most = octx > most ? octx : most;
+            }
+        }
+        const float mx = wave_max(static_cast<float>(most));
         const float mn = -wave_max(alive ? -static_cast<float>(ctx) : -static_cast<float>(max_len));
-        if (lane == 0) wmax[wave] = static_cast<uint32_t>(mx), wmax[kFlWaves + wave] = static_cast<uint32_t>(mn);
+        if (lane == 0) wmax[wave] = static_cast<uint32_t>(mx), wmax[W + wave] = static_cast<uint32_t>(mn);
     }
     // q of the pair as B fragments: dims 16 s + 8 h .. + 7
     uint4 qf[QS];
@@ -191,18 +208,17 @@ __global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_f
     __syncthreads();
     uint32_t kmax = 0, kmin = max_len;
 #pragma unroll
-    for (int w = 0; w < kFlWaves; ++w) {
+    for (int w = 0; w < W; ++w) {
         kmax = wmax[w] > kmax ? wmax[w] : kmax;
-        kmin = wmax[kFlWaves + w] < kmin ? wmax[kFlWaves + w] : kmin;
+        kmin = wmax[W + w] < kmin ? wmax[W + w] : kmin;
     }
-    if (kmax == 0) return;  // no live row (uniform over the block)
     const uint32_t trips = (kmax + C::kKeys - 1) / C::kKeys;
 
-    // trip it's keys into LDS by DMA: wavefront w brings kKeys / 8 of them in
+    // trip it's keys into LDS by DMA: wavefront w brings kKeys / W of them in
     // 1 KiB instructions (64 / PP keys x PP slots); keys past the block's
     // longest context read key kmax - 1 (valid, never used)
     const __amdgpu_buffer_rsrc_t rk = fl_rsrc(kc, static_cast<uint64_t>(max_len) * HD * 2);
-    constexpr uint32_t kPerWave = C::kKeys / kFlWaves, kPerInst = 64 / PP;
+    constexpr uint32_t kPerWave = C::kKeys / W, kPerInst = 64 / PP;
     auto stage_k = [&](uint32_t it, uint32_t buf) {
 #pragma unroll
         for (uint32_t c = 0; c < kPerWave / kPerInst; ++c) {
@@ -221,11 +237,11 @@ __global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_f
     // dims 8 c .. 8 c + 7, then writes dword (v[2i][d], v[2i+1][d]) of each
     // dim d to V^T
     constexpr uint32_t kVPairs = C::kKeys / 2, kVItems = kVPairs * PP;
-    constexpr int kVRounds = kVItems > kFlThreads ? kVItems / kFlThreads : 1;
+    constexpr int kVRounds = kVItems > C::kThreads ? kVItems / C::kThreads : 1;
     auto load_v = [&](uint32_t it, uint4 (&v)[kVRounds][2]) {
 #pragma unroll
         for (int r = 0; r < kVRounds; ++r) {
-            const uint32_t item = (tid + r * kFlThreads) % kVItems, i = item % kVPairs, c = item / kVPairs;
+            const uint32_t item = (tid + r * C::kThreads) % kVItems, i = item % kVPairs, c = item / kVPairs;
 #pragma unroll
             for (int e = 0; e < 2; ++e) {
                 uint32_t key = it * C::kKeys + 2 * i + e;
@@ -234,28 +250,19 @@ __global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_f
             }
         }
     };
-    auto specials = [](uint32_t x) {  // bit 15 / 31: that half is inf or NaN
-        return ((x & 0x7FFF7FFFu) + 0x00800080u) & 0x80008000u;
-    };
     // masked: some row does not attend all of the trip's keys
     auto store_v = [&](uint4 (&v)[kVRounds][2], uint32_t buf, bool masked) {
-        if (kVItems < kFlThreads && tid >= kVItems) return;
+        if (kVItems < C::kThreads && tid >= kVItems) return;
         if (masked) {
 #pragma unroll
             for (int r = 0; r < kVRounds; ++r) {
-                uint4 &x = v[r][0], &y = v[r][1];
-                if (specials(x.x) | specials(x.y) | specials(x.z) | specials(x.w) | specials(y.x) | specials(y.y) |
-                    specials(y.z) | specials(y.w)) {
-                    v_special = 1;
-                    auto clear = [&](uint32_t &w) { w &= ~((specials(w) >> 15) * 0xFFFFu); };
-                    clear(x.x), clear(x.y), clear(x.z), clear(x.w);
-                    clear(y.x), clear(y.y), clear(y.z), clear(y.w);
-                }
+                const bool x = clear_specials(v[r][0]), y = clear_specials(v[r][1]);
+                if (x || y) v_special = 1;
             }
         }
 #pragma unroll
         for (int r = 0; r < kVRounds; ++r) {
-            const uint32_t item = tid + r * kFlThreads, i = item % kVPairs, c = item / kVPairs;
+            const uint32_t item = tid + r * C::kThreads, i = item % kVPairs, c = item / kVPairs;
             uint16_t *const blk = vls + buf * C::kBuf + i / 32 * (kFlKeys * HD);
             const uint32_t slot = fl_slot(2 * (i % 32));  // even; key 2 i + 1 is the next slot
             const uint32_t a[4] = {v[r][0].x, v[r][0].y, v[r][0].z, v[r][0].w};
@@ -352,13 +359,13 @@ __global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_f
         meet(h ? mo : m, h ? lo : l, h ? m : mo, h ? l : lo, &M, &S);
         if constexpr (KS > 1) {
             float2 *const st = reinterpret_cast<float2 *>(wmax);  // [split][pair]
-            if (h == 0) st[split * C::kPairs + p] = make_float2(M, S);
+            if (h == 0) st[split * C::kPairs + pb] = make_float2(M, S);
             __syncthreads();
-            float2 v = st[p];
+            float2 v = st[pb];
             M = v.x, S = v.y;
 #pragma unroll
             for (int k = 1; k < KS; ++k) {
-                v = st[k * C::kPairs + p];
+                v = st[k * C::kPairs + pb];
                 meet(M, S, v.x, v.y, &M, &S);
             }
         }
@@ -464,7 +471,7 @@ __global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_f
     if (split == 0) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const uint32_t pp = pg * 32 + 8 * (r / 4) + 4 * h + (r % 4);
+            const uint32_t pp = p0 + pg * 32 + 8 * (r / 4) + 4 * h + (r % 4);
             if (pp >= LIVE || r0 + pp / G >= rows) continue;
             uint16_t *orow = out + (static_cast<uint64_t>(r0 + pp / G) * n_heads + h0 + pp % G) * HD + (lane & 31);
 #pragma unroll
@@ -477,102 +484,123 @@ __global__ __launch_bounds__(kFlThreads, HD == 64 && KS > 1 ? 4 : 2) void attn_f
     // the rows that attend the key, p from the score again
     __syncthreads();  // the outputs are written, the sums above read
     float2 *const st = reinterpret_cast<float2 *>(fl_smem);
-    if (split == 0 && h == 0) st[p] = make_float2(oM, S);
+    if (split == 0 && h == 0) st[pb] = make_float2(oM, S);
     __syncthreads();
-    for (uint32_t o = tid; o < LIVE * HD; o += kFlThreads) {
-        const uint32_t pp = o / HD, d = o % HD, row = r0 + pp / G;
-        if (row >= rows) continue;
+    for (uint32_t o = tid; o < C::kPairs * HD; o += C::kThreads) {
+        const uint32_t pi = o / HD, pp = p0 + pi, d = o % HD, row = r0 + pp / G;
+        if (pp >= LIVE || row >= rows) continue;
         const uint64_t at = (static_cast<uint64_t>(row) * n_heads + h0 + pp % G) * HD;
         const uint32_t rpos = positions[row], rctx = rpos < max_len ? rpos + 1 : max_len;
         float sum = 0.f;
         bool any = false;
         for (uint32_t j = kmin / C::kKeys * C::kKeys; j < rctx; ++j) {
             const uint32_t v = vc[static_cast<uint64_t>(j) * HD + d];
-            if (!specials(v)) continue;
+            if (!bf16_specials(v)) continue;
             float qk = 0.f;
             for (uint32_t e = 0; e < HD; ++e) qk = fmaf(bf(q[at + e]), bf(kc[k_offset(j, e, max_len, HD)]), qk);
-            sum += bf(rne(ex(bf(rne(qk)), st[pp].x) / st[pp].y)) * bf(static_cast<uint16_t>(v));
+            sum += bf(rne(ex(bf(rne(qk)), st[pi].x) / st[pi].y)) * bf(static_cast<uint16_t>(v));
             any = true;
         }
         if (any) out[at + d] = rne(bf(out[at + d]) + sum);
     }
 }
 
-// Over how many wavefronts the one-pass kernel splits the keys for `batch`
-// sequences of `rows` prompt rows (0: it does not take them): head_dim 64 or
-// 128, G = n_heads / n_kv of 1 .. 8, and query tiles for half the CUs or a
-// prompt of at least 16 rows that is not short against the cache, since a
-// block walks all of its rows' keys (from 1/11 of it, 1/16 for heads of 64).
-// Measured against the two-kernel path, 8 KV heads, 3 query heads each of
-// 128: 100 rows after 1000 keys 32.4 / 35.4 us, 48 after 500 21.4 / 20.4, 48
-// after 2000 50.1 / 37.2, 512 alone 23.5 / 36.5; heads of 64: 24 after 300
-// 10.9 / 14.9, 2048 after 1024 108 / 603.8. The maximum is taken before the
-// scale, which has to be positive, and contexts are compared as floats and
-// keys addressed by 32-bit byte offsets: caches below 2^24 keys.
-// No split where the batch's blocks make two rounds of CUs (8 x 2048 rows, two
-// layers' prompt 14.22 ms against 14.53 over 2 and 15.35 over 4); else over 2
-// where that gives more than a block per CU, 4 otherwise: one 2048-row prompt
-// (256 blocks unsplit, which wait for the one with the most keys) 130.5, 99.4
-// and 135.4 us over 1, 2 and 4, 512 rows 34.8, 23.5 and 19.3. Longer prompts
-// with heads of 128 stay at 2 all the same: the error against 64 bits is the
-// same at 2 and 4, but over 4 the rounding of a 28-layer model's 512-row prompt
-// moved its second greedy id, a near tie, out of the reference's top 5.
-uint32_t attention_flash_splits(uint32_t cus, uint32_t batch, uint32_t rows, uint32_t n_heads, uint32_t n_kv,
-                                uint32_t head_dim, uint32_t max_len, float scale) {
-    if (!(scale > 0.f && scale * 1.5f < INFINITY) || max_len >= 1u << 24) return 0;
-    if ((head_dim != 64 && head_dim != 128) || n_kv == 0 || n_heads % n_kv != 0) return 0;
+// The block shape the one-pass kernel takes for `batch` sequences of `rows`
+// prompt rows (waves = 0: it does not take them). Whether it does, and over how
+// many wavefronts a pair's keys are split, goes by one sequence alone, so a
+// batch gives what a call per sequence gives.
+struct FlPlan {
+    uint32_t waves = 0, ks = 1;
+};
+
+static FlPlan flash_plan(uint32_t cus, uint32_t batch, uint32_t rows, uint32_t n_heads, uint32_t n_kv,
+                         uint32_t head_dim, uint32_t max_len, float scale) {
+    FlPlan p;
+    // the maximum is taken before the scale, which has to be positive; contexts
+    // are compared as floats and keys addressed by 32-bit byte offsets
+    if (!(scale > 0.f && scale * 1.5f < INFINITY) || max_len >= 1u << 24) return p;
+    if ((head_dim != 64 && head_dim != 128) || n_kv == 0 || n_heads % n_kv != 0) return p;
     const uint32_t g = n_heads / n_kv;
-    if (g < 1 || g > 8) return 0;
-    auto blocks = [&](uint32_t ks) {  // of one sequence
-        const uint32_t qt = 256 / ks / g;
-        return (static_cast<uint64_t>(rows) + qt - 1) / qt * n_kv;
-    };
-    if (2 * blocks(1) < cus && (rows < 16 || max_len > static_cast<uint64_t>(head_dim == 64 ? 16 : 11) * rows)) return 0;
-    const uint32_t ks = blocks(1) * batch >= 2ull * cus ? 1
-                        : blocks(2) > cus || (head_dim == 128 && rows >= 256) ? 2 : 4;
-    return blocks(ks) / n_kv > 65535 ? 0 : ks;
+    if (g < 1 || g > 8) return p;
+    auto tiles = [&](uint32_t pairs) { return (static_cast<uint64_t>(rows) + pairs / g - 1) / (pairs / g); };
+    const uint64_t blocks = tiles(256) * n_kv;  // of one sequence, in blocks of 256 pairs
+    if (head_dim == 128) {
+        // Query tiles for half the CUs. Below that the two-kernel path: 512
+        // rows of 24 heads, 8 KV heads, take 36.1 us there and 34.8 here. (With
+        // the keys split over wavefronts they take 24.7, but then round the
+        // sums otherwise, and a prompt's logits move by 3.5e-4.)
+        if (2 * blocks < cus || tiles(256) > 65535) return p;
+        // Blocks of 4 wavefronts where 8 would not make two rounds of CUs: two
+        // share a CU, so one with few keys can run beside one with many. 8 KV
+        // heads, in blocks of 8 and 4: 2048 rows of 32 heads 126.8 / 105.9 us
+        // (after 1024 189.7 / 165.0), 1024 rows 64.8 / 50.2.
+        p.waves = blocks * batch >= 2ull * cus ? 8 : 4;
+        return p;
+    }
+    // Query tiles for half the CUs, or a prompt of at least 16 rows that is not
+    // short against the cache, since a block walks all of its rows' keys.
+    // Measured against the two-kernel path, 32 heads, 8 KV heads: 24 rows after
+    // 300 keys 10.9 / 14.9 us, 2048 after 1024 108 / 603.8. The keys over 2
+    // wavefronts where that gives more than a block per CU, 4 otherwise, none
+    // from two rounds on.
+    if (2 * blocks < cus && (rows < 16 || max_len > 16ull * rows)) return p;
+    p.ks = blocks >= 2ull * cus ? 1 : tiles(128) * n_kv > cus ? 2 : 4;
+    p.waves = tiles(256 / p.ks) > 65535 ? 0 : 8;
+    return p;
 }
 
-template <int HD, int G, int KS>
+// Whether fh_attention takes the one-pass kernel for `rows` prompt rows of a
+// sequence.
+bool attention_flash_applies(uint32_t cus, uint32_t rows, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
+                             uint32_t max_len, float scale) {
+    return flash_plan(cus, 1, rows, n_heads, n_kv, head_dim, max_len, scale).waves != 0;
+}
+
+template <int HD, int G, int W, int KS>
 static void launch_flash(hipStream_t stream, const uint16_t *q, const uint32_t *positions, uint32_t rows,
                          const uint16_t *k_cache, const uint16_t *v_cache, uint32_t n_heads, uint32_t n_kv,
                          uint32_t max_len, float scale, uint16_t *out, uint32_t batch, uint64_t seq_cache) {
-    using C = FlCfg<HD, KS>;
+    using C = FlCfg<HD, W, KS>;
     static const hipError_t opt_in =
-        hipFuncSetAttribute(reinterpret_cast<const void *>(attn_flash_kernel<HD, G, KS>),
+        hipFuncSetAttribute(reinterpret_cast<const void *>(attn_flash_kernel<HD, G, W, KS>),
                             hipFuncAttributeMaxDynamicSharedMemorySize, C::kLds);
     (void)opt_in;
-    constexpr uint32_t QT = C::kPairs / G;
-    hipLaunchKernelGGL((attn_flash_kernel<HD, G, KS>), dim3(n_kv, batch, (rows + QT - 1) / QT), dim3(kFlThreads),
-                       C::kLds, stream, q, positions, rows, k_cache, v_cache, seq_cache, n_heads, max_len, scale, out);
+    constexpr uint32_t QT = C::kPairs * C::kParts / G;
+    hipLaunchKernelGGL((attn_flash_kernel<HD, G, W, KS>), dim3(n_kv, batch, (rows + QT - 1) / QT * C::kParts),
+                       dim3(C::kThreads), C::kLds, stream, q, positions, rows, k_cache, v_cache, seq_cache, n_heads,
+                       max_len, scale, out);
 }
 
 // Launches the one-pass kernel over `batch` sequences of `rows` rows (q, out
 // and positions consecutive per sequence, caches seq_cache elements apart)
-// when attention_flash_splits takes them; returns false otherwise (the caller
-// takes the two-kernel path). Where one sequence alone splits its keys alike,
-// every block is the one a launch per sequence would run.
+// when attention_flash_applies; returns false otherwise (the caller takes the
+// two-kernel path). The outputs are those of a launch per sequence.
 bool launch_attention_flash(hipStream_t stream, uint32_t cus, const uint16_t *q, const uint32_t *positions,
                             uint32_t rows, const uint16_t *k_cache, const uint16_t *v_cache, uint32_t n_heads,
                             uint32_t n_kv, uint32_t head_dim, uint32_t max_len, float scale, uint16_t *out,
                             uint32_t batch, uint64_t seq_cache) {
-    const uint32_t ks = attention_flash_splits(cus, batch, rows, n_heads, n_kv, head_dim, max_len, scale);
-    if (batch == 0 || batch > 65535 || ks == 0) return false;
+    if (batch == 0 || batch > 65535) return false;
+    const FlPlan p = flash_plan(cus, batch, rows, n_heads, n_kv, head_dim, max_len, scale);
+    if (p.waves == 0) return false;
     const uint32_t g = n_heads / n_kv;
-#define FH_FLASH(HH, GG, SS)                                                                                  \
-    if (head_dim == HH && g == GG && ks == SS) {                                                              \
-        launch_flash<HH, GG, SS>(stream, q, positions, rows, k_cache, v_cache, n_heads, n_kv, max_len, scale, \
-                                 out, batch, seq_cache);                                                      \
-        return true;                                                                                          \
+#define FH_FLASH(HH, GG, WW, SS)                                                                                  \
+    if (head_dim == HH && g == GG && p.waves == WW && p.ks == SS) {                                               \
+        launch_flash<HH, GG, WW, SS>(stream, q, positions, rows, k_cache, v_cache, n_heads, n_kv, max_len, scale, \
+                                     out, batch, seq_cache);                                                      \
+        return true;                                                                                              \
     }
-#define FH_FLASH_KS(HH, GG) FH_FLASH(HH, GG, 1) FH_FLASH(HH, GG, 2) FH_FLASH(HH, GG, 4)
-#define FH_FLASH_G(HH)                                                                        \
-    FH_FLASH_KS(HH, 1) FH_FLASH_KS(HH, 2) FH_FLASH_KS(HH, 3) FH_FLASH_KS(HH, 4) FH_FLASH_KS(HH, 5) \
-    FH_FLASH_KS(HH, 6) FH_FLASH_KS(HH, 7) FH_FLASH_KS(HH, 8)
-    FH_FLASH_G(64)
-    FH_FLASH_G(128)
+#define FH_FLASH_G(GG)                                                       \
+    FH_FLASH(64, GG, 8, 1) FH_FLASH(64, GG, 8, 2) FH_FLASH(64, GG, 8, 4)     \
+    FH_FLASH(128, GG, 8, 1) FH_FLASH(128, GG, 4, 1)
+    FH_FLASH_G(1)
+    FH_FLASH_G(2)
+    FH_FLASH_G(3)
+    FH_FLASH_G(4)
+    FH_FLASH_G(5)
+    FH_FLASH_G(6)
+    FH_FLASH_G(7)
+    FH_FLASH_G(8)
 #undef FH_FLASH_G
-#undef FH_FLASH_KS
 #undef FH_FLASH
     return false;
 }

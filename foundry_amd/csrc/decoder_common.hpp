@@ -129,6 +129,19 @@ __device__ __forceinline__ float wave_max(float v) {
     return fmaxf(fmaxf(lane_value(v, 0), lane_value(v, 16)), fmaxf(lane_value(v, 32), lane_value(v, 48)));
 }
 
+// Bit 15 / 31 where that half of x is a bf16 inf or NaN.
+__device__ __forceinline__ uint32_t bf16_specials(uint32_t x) {
+    return ((x & 0x7FFF7FFFu) + 0x00800080u) & 0x80008000u;
+}
+
+// Sets the infs and NaNs among 8 bf16 to 0; true if there were any.
+__device__ __forceinline__ bool clear_specials(uint4 &v) {
+    if ((bf16_specials(v.x) | bf16_specials(v.y) | bf16_specials(v.z) | bf16_specials(v.w)) == 0) return false;
+    auto clear = [](uint32_t &w) { w &= ~((bf16_specials(w) >> 15) * 0xFFFFu); };
+    clear(v.x), clear(v.y), clear(v.z), clear(v.w);
+    return true;
+}
+
 // RoPE (src/models/llama/rotary_emb.rs:62-85) of dims p*8 .. p*8+7 of one
 // head: x' = RNE(RNE(x * cos) + RNE(rot * sin)), rot = cat(-x2, x1); the
 // partner piece is the matching 8 dims of the other half (hp pieces per

@@ -29,8 +29,8 @@ void launch_silu_mul_partials(hipStream_t stream, const float *part, uint32_t sp
 bool launch_q4_gemm_direct_silu(hipStream_t stream, uint32_t cus, const uint16_t *x, uint32_t x_ld,
                                 const uint32_t *wq, const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t f,
                                 uint32_t k, uint16_t *act);
-uint32_t attention_flash_splits(uint32_t cus, uint32_t batch, uint32_t rows, uint32_t n_heads, uint32_t n_kv,
-                                uint32_t head_dim, uint32_t max_len, float scale);
+bool attention_flash_applies(uint32_t cus, uint32_t rows, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
+                             uint32_t max_len, float scale);
 bool launch_attention_flash(hipStream_t stream, uint32_t cus, const uint16_t *q, const uint32_t *positions,
                             uint32_t rows, const uint16_t *k_cache, const uint16_t *v_cache, uint32_t n_heads,
                             uint32_t n_kv, uint32_t head_dim, uint32_t max_len, float scale, uint16_t *out,
@@ -257,15 +257,14 @@ int attention(fh_device *d, const fh_llama_model &m, const fh_llama_layer &L, in
     const int64_t hq = m.n_heads * m.head_dim;
     const int64_t qkv_n = (m.n_heads + 2 * m.n_kv_heads) * m.head_dim;
     const int64_t seq_cache = m.n_kv_heads * m.max_len * m.head_dim;  // one sequence's cache, elements
-    // where the one-pass kernel takes the sequences they share one launch of
-    // it, longest blocks first across the batch (a large batch may split its
-    // keys over fewer wavefronts than one sequence's call would)
+    // where each sequence's call would take the one-pass kernel, the
+    // sequences share one launch of it (the same sums, longest blocks first
+    // across the batch)
     const bool one_launch =
         m.batch > 1 && m.batch <= 65535 && m.max_len <= 0xFFFFFFFFll &&
-        fh::attention_flash_splits(d->compute_units, static_cast<uint32_t>(m.batch),
-                                   static_cast<uint32_t>(seq_tokens), static_cast<uint32_t>(m.n_heads),
-                                   static_cast<uint32_t>(m.n_kv_heads), static_cast<uint32_t>(m.head_dim),
-                                   static_cast<uint32_t>(m.max_len), m.scale) != 0 &&
+        fh::attention_flash_applies(d->compute_units, static_cast<uint32_t>(seq_tokens),
+                                    static_cast<uint32_t>(m.n_heads), static_cast<uint32_t>(m.n_kv_heads),
+                                    static_cast<uint32_t>(m.head_dim), static_cast<uint32_t>(m.max_len), m.scale) &&
         aligned16(m.q) && aligned16(m.attn) && aligned16(L.k_cache) && aligned16(L.v_cache);
     // the RoPE and cache writes of every sequence in one launch
     const float *part = qkv_splits > 1 ? static_cast<const float *>(d->partial_area) : nullptr;

@@ -552,7 +552,7 @@ typedef struct fh_llama_model {
  * the ops above one by one: up to 8 rows the RMSNorms, residual adds and SiLU
  * go inside the GEMVs and one new token's RoPE and cache write inside
  * fh_decode_attention; above 8 rows the unfused ops run, and prefill
- * attention runs one sequence at a time. Above 8 rows a GEMM that splits K
+ * attention gives what fh_attention gives for each sequence alone. Above 8 rows a GEMM that splits K
  * passes its f32 partials (the device's partial area) to the RoPE, RMSNorm
  * or SiLU after it, which adds them in the order of the GEMM's own reduce:
  * the results are bit-identical to the op sequence, but the buffers o,

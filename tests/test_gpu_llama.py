@@ -223,11 +223,12 @@ def test_attention_one_pass_prefill(device, n_heads, n_kv, t, max_len, past):
     assert np.array_equal(got, again), "one-pass attention differs between runs"
 
 
-# The one-pass kernel's key splits: 4 (few query tiles: ragged last tiles, one
-# trip of keys, a context that ends inside a wavefront's run of keys, groups of
-# 7 and 8 heads), 2 (a block per CU) and none (two rounds), head sizes 64 and
-# 128, and prompts too short against their cache, which the two-kernel path
-# keeps. One position lies past the cache (it attends all of it).
+# The one-pass kernel's forms: heads of 64 with their keys over 4 wavefronts
+# (few query tiles: a ragged last tile), 2 (more than a block per CU) and none
+# (two rounds), heads of 128 in blocks of 4 wavefronts; and the two-kernel path
+# beside it, for short prompts with heads of 128 (one trip of keys, groups of 7
+# and 8 heads) and prompts too short against their cache. One position lies
+# past the cache (it attends all of it).
 FLASH_SPLIT_CASES = [(32, 8, 64, 40, 100, 50), (32, 8, 64, 700, 901, 201), (32, 8, 64, 1100, 1190, 90),
                      (64, 64, 64, 2048, 2060, 12), (4, 2, 128, 16, 16, 0), (24, 8, 128, 100, 161, 61),
                      (14, 2, 128, 130, 1030, 900), (16, 2, 128, 65, 97, 32), (32, 8, 128, 1024, 1088, 64),
@@ -251,10 +252,13 @@ def test_attention_one_pass_key_splits(device, n_heads, n_kv, hd, t, max_len, pa
 
 
 # inf and NaN of V reach only the rows that attend their keys, and only in
-# their dim (KS 4, 2 and none; positions out of order, so that many trips hold
-# keys that only some rows attend)
+# their dim (heads of 64 with their keys over 4, 2 and 1 wavefronts; the
+# two-kernel path's query-row tiles with P.V in one chunk and in several, ragged
+# last tiles of 3 and 16 rows; blocks of 4 and 8 wavefronts; positions out of
+# order, so that many trips hold keys that only some rows attend)
 @pytest.mark.parametrize("n_heads,n_kv,hd,t,past", [(32, 8, 64, 70, 30), (8, 2, 128, 200, 0), (32, 8, 64, 1100, 0),
-                                                    (64, 64, 64, 2048, 0)])
+                                                    (64, 64, 64, 2048, 0), (24, 8, 128, 512, 0), (4, 4, 128, 23, 900),
+                                                    (32, 8, 128, 1100, 0), (64, 64, 128, 2048, 0)])
 def test_attention_one_pass_special_values(device, n_heads, n_kv, hd, t, past):
     max_len = past + t
     q = synth.bf16_normal(41, (t, n_heads, hd))
@@ -779,7 +783,21 @@ def test_llama_forward_one_attention_launch_for_the_batch(device, depth):
     per sequence). depth: the second sequence's rows sit that many positions
     further on (its cache below them zero, as allocated), so each sequence's
     positions and cache are its own in the shared launch."""
-    batch, t, c = 2, 1024, FLASH
+    _batch_forward_equals_ops(device, FLASH, 1024, depth)
+
+
+# Prompts whose blocks make two rounds of CUs as a batch of two, but not alone:
+# 4, 3 and 7 heads of 128 per KV head (a call per sequence takes blocks of 4
+# wavefronts, the batch of 8), and heads of 64 (keys over 2 wavefronts alone)
+@pytest.mark.parametrize("n_heads,n_kv,hd,t", [(32, 8, 128, 2048), (24, 8, 128, 2900), (14, 2, 128, 4700),
+                                               (32, 8, 64, 2048)])
+def test_llama_forward_long_prompts_of_a_batch(device, n_heads, n_kv, hd, t):
+    c = LlamaConfig(n_layers=1, hidden=1024, n_heads=n_heads, n_kv_heads=n_kv, head_dim=hd, ffn=1024, vocab=1000)
+    _batch_forward_equals_ops(device, c, t, 100)
+
+
+def _batch_forward_equals_ops(device, c, t, depth):
+    batch = 2
     model = Q4Llama(device, c, 6, t + depth, max_tokens=t, batch=batch)
     b = model.buf
     model._upload(b["ids"], np.ascontiguousarray(synth.token_ids(12, batch * t, c.vocab), dtype=np.uint32))
