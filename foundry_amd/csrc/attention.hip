@@ -781,11 +781,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
     constexpr uint32_t R = 16 / G, LIVE = R * G;
     constexpr int DT = HD / 16;  // 16-dim tiles of the output
     static_assert(HD == 128, "a lane transposes 8 keys x 8 dims, 16 pieces per key row");
-    static_assert(sizeof(uint16_t) * kAttnWaves * HD * kPvtPitch >= sizeof(float) * kAttnWaves * 16 * HD,
-                  "the wavefronts' sums fit the transposed-V area");
+    static_assert(sizeof(uint16_t) * kAttnWaves * HD * kPvtPitch >= sizeof(float) * kAttnWaves * 16 * HD + 256,
+                  "the wavefronts' sums, the rows' M and S and four flags fit the transposed-V area");
     __shared__ __align__(16) uint16_t vt[kAttnWaves][HD][kPvtPitch];
-    __shared__ uint32_t special[kAttnWaves];  // a wavefront staged an inf or NaN as 0
-    __shared__ float2 row_ms[16];
     const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, col = lane & 15, quad = lane >> 4;
     const uint32_t kvh = blockIdx.x / chunks, c = blockIdx.x % chunks;
     const uint32_t r0 = blockIdx.y * R, h0 = kvh * G;
@@ -852,7 +850,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
     uint16_t(*vw)[kPvtPitch] = vt[wave];
     uint4 va[8];
     float sa[8];
-    bool cleared = false;
+    bool cleared = false;  // the same in every lane
     uint32_t s = wave;
     if (s < nsteps) {
         load_v(s, va);
@@ -866,10 +864,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
             load_v(s + kAttnWaves, vn);
             load_s(s + kAttnWaves, sn);
         }
-        if (k0 + s * 32 + 32 > cmin) {  // some row does not attend all of the step's keys
-#pragma unroll
-            for (int t = 0; t < 8; ++t) cleared |= clear_specials(va[t]);
-        }
+        const bool partly = k0 + s * 32 + 32 > cmin;  // some row does not attend all of the step's keys
         // transpose: dim 8 pv + d of keys 8 vj .. 8 vj + 7 as one 16-byte row piece
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
@@ -881,7 +876,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
                 const uint32_t bw = d / 2 == 0 ? b.x : d / 2 == 1 ? b.y : d / 2 == 2 ? b.z : b.w;
                 w[i] = d % 2 ? (aw >> 16) | (bw & 0xFFFF0000u) : (aw & 0xFFFFu) | (bw << 16);
             }
-            *reinterpret_cast<uint4 *>(&vw[8 * pv + d][8 * vj]) = make_uint4(w[0], w[1], w[2], w[3]);
+            uint4 piece = make_uint4(w[0], w[1], w[2], w[3]);
+            if (partly) cleared |= __any(clear_specials(piece)) != 0;
+            *reinterpret_cast<uint4 *>(&vw[8 * pv + d][8 * vj]) = piece;
         }
         // A: the probabilities of keys 8 quad .. 8 quad + 7 of the step for this lane's row
         const uint32_t kb = k0 + s * 32 + 8 * quad;
@@ -907,13 +904,16 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
             for (int e = 0; e < 8; ++e) sa[e] = sn[e];
         }
     }
-    const uint32_t wave_cleared = __any(cleared) ? 1u : 0u;
-    if (lane == 0) special[wave] = wave_cleared;
-    if (wave == 0 && quad == 0) row_ms[col] = make_float2(mrow, srow_sum);
     // the wavefronts' sums, added in wavefront order: result lane (dim col of
     // tile t, row quad) holds rows 4 quad + i
     __syncthreads();  // every wavefront is done with its V slice
     float(*red)[16][HD] = reinterpret_cast<float(*)[16][HD]>(&vt[0][0][0]);
+    // behind the sums (four blocks a CU need every byte): M and S of the rows,
+    // and whether a wavefront staged an inf or NaN as 0
+    float2 *const row_ms = reinterpret_cast<float2 *>(&red[kAttnWaves][0][0]);
+    uint32_t *const special = reinterpret_cast<uint32_t *>(row_ms + 16);
+    if (lane == 0) special[wave] = cleared ? 1u : 0u;
+    if (wave == 0 && quad == 0) row_ms[col] = make_float2(mrow, srow_sum);
 #pragma unroll
     for (int t = 0; t < DT; ++t)
 #pragma unroll
