@@ -332,9 +332,13 @@ static double tiled_gemm_us(uint32_t cus, uint32_t x_ld, uint32_t m, uint32_t n,
 //   kernels' by 3% (both models above and there; measured, rows kernel
 //   against 256-row kernels: 32 x 28672 x 4096 27.2 against 75.8 us, 48 x 4096
 //   x 4096 8.8 / 20.5, 128 x 5120 x 3072 13.2 / 25.7, 256 x 3072 x 8192 24.1 /
-//   35.4, 512 x 3072 x 3072 21.8 / 29.5, 1024 x 3072 x 8192 88.2 / 101.5; on
-//   the other side of the line 1024 x 5120 x 3072 70.1 / 66.2, 256 x 16384 x
-//   3072 57.1 / 51.1);
+//   35.4; on the other side of the line 256 x 16384 x 3072 57.1 / 51.1). From
+//   512 rows, two whole 256-row tiles, only where it is below by 30%: it adds
+//   a sum over K in eight parts, which moves a prompt's logits (two layers of
+//   hidden 3072, 512 rows, by 3e-4 with the attention beside it), and most
+//   prompts gain little from it (512 x 5120 x 3072 33.4 / 34.8 us, 512 x 3072 x
+//   3072 21.8 / 29.5, 1024 x 5120 x 3072 70.1 / 66.2). Narrow weights pass the
+//   line (512 x 2048 x 2048);
 // - weights straight to the matrix cores (q4_gemm_direct.hip) where its
 //   256 x 256 tiles fill the chip, or 3/4 of it over two K ranges;
 // - q4_gemm_kernel otherwise.
@@ -346,7 +350,7 @@ uint32_t launch_q4_gemm_deferred(hipStream_t stream, uint32_t cus, const uint16_
                                  const uint32_t *wq, const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t n,
                                  uint32_t k, void *y, int y_is_f32, void *area) {
     const RowsPlan rows = plan_q4_gemm_rows(cus, x_ld, s, b, m, n, k);
-    if (rows.ct != 0 && 1.03 * rows.us < tiled_gemm_us(cus, x_ld, m, n, k, area != nullptr)) {
+    if (rows.ct != 0 && rows.us * (m < 512 ? 1.03 : 1.43) < tiled_gemm_us(cus, x_ld, m, n, k, area != nullptr)) {
         launch_q4_gemm_rows(stream, rows, x, x_ld, wq, s, b, m, n, k, y, y_is_f32);
         return 1;
     }

@@ -702,20 +702,51 @@ def _op_by_op_forward(model, seq_tokens):
     call("fh_argmax", d, P(b["logits"]), model.batch, c.vocab, P(b["next"]))
 
 
-# hidden 512 and FFN 1024: the q/k/v, o, gate/up and down GEMMs of these row
-# counts split K (2, 2, 2 and 4 splits), so fh_llama_forward's RoPE, norms
-# and SiLU form their inputs from the partials
+# hidden 512 and FFN 1024: GEMMs of the few-row kernel at these row counts
 SPLIT = LlamaConfig(n_layers=2, hidden=512, n_heads=8, n_kv_heads=2, head_dim=64, ffn=1024, vocab=1000)
 
 
 @pytest.mark.parametrize("batch,t", [(2, 20), (1, 300), (12, 1)])
 def test_llama_forward_equals_the_op_sequence(device, batch, t):
-    """fh_llama_forward above 8 rows (split GEMMs feeding the RoPE, norms
-    and SiLU; 12 sequences of one token: unfused ops around the decode
-    attention) gives bit-identical logits, hidden states and next ids to
-    the same forward issued op by op."""
-    model = Q4Llama(device, SPLIT, 5, 512, max_tokens=t, batch=batch)
-    b, c = model.buf, SPLIT
+    """fh_llama_forward above 8 rows (12 sequences of one token: unfused ops
+    around the decode attention) gives bit-identical logits, hidden states and
+    next ids to the same forward issued op by op."""
+    _forward_equals_ops(device, Q4Llama(device, SPLIT, 5, 512, max_tokens=t, batch=batch), batch, t)
+
+
+# GEMMs that split K, whose f32 partials the RoPE, norms and SiLU after them
+# add: widths of an odd number of 64-value groups (2, 2, 2 and 4 splits; the
+# few-row kernel takes whole pairs of groups) at few rows, and a 512-row prompt
+# at hidden 3072 (3, 6, 2 and 5 splits)
+ODD = LlamaConfig(n_layers=2, hidden=576, n_heads=9, n_kv_heads=3, head_dim=64, ffn=1088, vocab=1000)
+WHOLE = LlamaConfig(n_layers=1, hidden=3072, n_heads=24, n_kv_heads=8, head_dim=128, ffn=8192, vocab=1000)
+
+
+@pytest.mark.parametrize("cfg,batch,t", [(ODD, 2, 20), (ODD, 1, 300), (ODD, 12, 1), (WHOLE, 1, 512)])
+def test_llama_forward_with_split_gemms(device, cfg, batch, t):
+    """fh_llama_forward adds a split GEMM's partials inside the op that
+    consumes it: the buffers o and gate_up, and for prompts qkv, are then not
+    written (so a dispatch that no longer splits fails here), and logits,
+    hidden states and next ids are those of the op sequence, bit for bit."""
+    model = Q4Llama(device, cfg, 5, 512, max_tokens=t, batch=batch)
+    sizes = {"o": cfg.hidden, "gu": 2 * cfg.ffn, "qkv": cfg.qkv_rows}
+    if t == 1:
+        del sizes["qkv"]
+    marks = {name: np.full(batch * t * width, 0x7FC1, np.uint16) for name, width in sizes.items()}
+
+    def before():
+        for name, mark in marks.items():
+            model._upload(model.buf[name], mark)
+
+    def after():
+        for name, mark in marks.items():
+            assert np.array_equal(down(device, model.buf[name], np.uint16, mark.size), mark), name
+
+    _forward_equals_ops(device, model, batch, t, before, after)
+
+
+def _forward_equals_ops(device, model, batch, t, before=lambda: None, after=lambda: None):
+    b, c = model.buf, model.cfg
     ids = synth.token_ids(11, batch * t, c.vocab).reshape(batch, t)
     model._upload(b["ids"], np.ascontiguousarray(ids, dtype=np.uint32))
     model._upload(b["positions"], np.tile(np.arange(t, dtype=np.uint32), batch))
@@ -725,7 +756,9 @@ def test_llama_forward_equals_the_op_sequence(device, batch, t):
         return (down(device, b["logits"], np.uint16, batch * c.vocab), down(device, b["h"], np.uint16, rows * c.hidden),
                 down(device, b["next"], np.uint32, batch))
 
+    before()
     model._forward(t, b["ids"], b["positions"])
+    after()
     native = state()
     _op_by_op_forward(model, t)
     ops = state()

@@ -322,8 +322,10 @@ def test_gemm_split_ranges_sampled_and_repeatable(device, oracle, m, n, k):
 # Prompt-length rows whose tiles leave CUs idle split K (up to 8 ranges of
 # at least 4 steps, f32 partials added in order): the config-4 prefill's
 # down (5 splits) and q/k/v (3 splits) shapes, and m * n not a multiple of 4
-# (the reduce's scalar tail).
-@pytest.mark.parametrize("m,n,k", [(512, 3072, 8192), (512, 5120, 3072), (35, 198, 2048)])
+# (the reduce's scalar tail) where the few-row kernel does not take the shape,
+# k an odd multiple of 64; (35, 198, 2048) is one it takes.
+@pytest.mark.parametrize("m,n,k", [(512, 3072, 8192), (512, 5120, 3072), (35, 198, 2048), (35, 198, 2112),
+                                   (515, 199, 2112)])
 def test_gemm_split_k(device, oracle, m, n, k):
     run_linear(device, oracle, m, n, k, seed=5000 + m + n, sample=(64, n) if m > 64 else None)
 
