@@ -369,9 +369,10 @@ __global__ __launch_bounds__(64 * W, HD == 64 && KS > 1 ? 4 : 2) void attn_flash
                 meet(M, S, v.x, v.y, &M, &S);
             }
         }
-        if (M == -INFINITY) S = 1.f;
+        // every score -inf: exp(-inf + inf) is NaN for a live pair; a dead lane,
+        // with no key, gets exp(-inf) = 0 everywhere
+        if (M == -INFINITY) S = alive ? NAN : 1.f;
     }
-    // a pair with no key (a dead lane) gets exp(-inf) = 0 everywhere, not NaN
     const float oM = M == -INFINITY ? 0.f : ex.base(M);
 #if FH_FLASH_RCP
     const float rS = 1.f / S;

@@ -287,6 +287,45 @@ def test_attention_one_pass_special_values(device, n_heads, n_kv, hd, t, past):
     assert np.array_equal(got[~hit], clean[~hit])
 
 
+# Scores of -inf, inf and NaN, on the one-pass kernel (heads of 64 with their
+# keys over 4, 2 and 1 wavefronts, blocks of 4 and 8) and the two-kernel path
+@pytest.mark.parametrize("n_heads,n_kv,hd,t", [(32, 8, 64, 70), (32, 8, 64, 1100), (64, 64, 64, 2048),
+                                               (24, 8, 128, 100), (32, 8, 128, 1100), (64, 64, 128, 2048)])
+def test_attention_special_scores(device, n_heads, n_kv, hd, t):
+    """A row whose every score is -inf, or that holds a NaN or +inf score, is
+    NaN, as softmax gives it; a key with a score of -inf beside finite ones
+    has weight 0, and the rows and heads that see none of these keep their
+    bits."""
+    g = n_heads // n_kv
+    q = synth.bf16_normal(61, (t, n_heads, hd))
+    kc = synth.bf16_normal(62, (n_kv, t, hd))
+    vc = synth.bf16_normal(63, (n_kv, t, hd))
+    pos = np.arange(t)
+    q[:, :, 0] = synth.bf16_rne(np.abs(R.from_bf16(q[:, :, 0])) + np.float32(0.25))  # dim 0 of every query is positive
+    clean, scale, _ = run_attention(device, q, kc, vc, pos)
+    bad = t // 2 + 3
+    kc[0, 0, 0] = 0xFF80  # key 0 of KV head 0: -inf
+    kc[1, bad, 3] = 0x7FC0  # a key of KV head 1: NaN
+    row, head = t // 3, n_heads - 1  # one query all -inf, its neighbour all +inf
+    kc[n_kv - 1, :, 1] = synth.bf16_rne(-np.abs(R.from_bf16(kc[n_kv - 1, :, 1])) - np.float32(0.25))
+    base, _, _ = run_attention(device, q, kc, vc, pos)
+    q[row, head, 1], q[row + 1, head, 1] = 0x7F80, 0xFF80
+    got, _, _ = run_attention(device, q, kc, vc, pos)
+    nan = np.isnan(R.from_bf16(got))
+    want = np.zeros(got.shape, dtype=bool)
+    want[0, :g] = True
+    want[bad:, g:2 * g] = True
+    want[row, head] = want[row + 1, head] = True
+    assert np.array_equal(nan, want), np.argwhere(nan != want)[:4].tolist()
+    rows = [1, 2, t // 2, t - 1]
+    ref, flip = attention_ref(q[:, :g], kc[:1], vc[:1], pos, scale, rows)
+    assert_attention_close(got[rows, :g], ref[rows], flip[rows], rows)
+    assert np.array_equal(got[:bad, g:2 * g], clean[:bad, g:2 * g])
+    keep = ~want
+    keep[:, :g] = False
+    assert np.array_equal(got[keep], base[keep])
+
+
 # scales the one-pass kernel does not take: equal weights at 0, and the lowest
 # scores first below it
 @pytest.mark.parametrize("scale", [0.0, -0.125])
