@@ -131,6 +131,7 @@ SIGNATURES = {
     "fh_alloc": [_vp, _sz, _int, ctypes.POINTER(_vp)],
     "fh_alloc_output": [_vp, _sz, ctypes.POINTER(_vp)],
     "fh_free": [_vp, _vp],
+    "fh_free_ordered": [_vp, _vp],
     "fh_upload": [_vp, _vp, _vp, _sz],
     "fh_download": [_vp, _vp, _vp, _sz],
     "fh_max_memory_allocated": [_vp, ctypes.POINTER(AllocatedMemory)],

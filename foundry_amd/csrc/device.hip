@@ -170,12 +170,14 @@ static hipError_t trim_pool(fh_device *dev, size_t count) {
 
 // Releases an allocation that is no longer in dev->allocs and that no live
 // graph uses. Up to kPoolBlockBytes it is kept for a later fh_alloc (oldest
-// kept blocks make room), else freed once the stream's work ends. Every op
-// returns fresh storage, so a program that runs op by op allocates and frees
-// once per op: through the driver that was two host-device round trips an op
-// (14 ops of attention over 512 tokens: 2.72 ms a pass for 0.4 ms of
-// kernels); from kept blocks a pass takes 0.36 ms.
-static hipError_t release(fh_device *dev, uintptr_t base, size_t size) {
+// kept blocks make room), else freed. Unless `ordered` says that only ops on
+// the device's stream have touched it, the caller may still be using it on a
+// stream of its own: take_pooled then waits before it goes out again. Every op
+// returns fresh storage, so a program that runs op
+// by op allocates and frees once per op: through the driver that was two
+// host-device round trips an op (14 ops of attention over 512 tokens: 2.5 ms a
+// pass for 0.15 ms of kernels); from kept blocks a pass takes 0.28 ms.
+static hipError_t release(fh_device *dev, uintptr_t base, size_t size, bool ordered) {
     dev->live_bytes -= size;
     const size_t cap = dev->capacity[base];
     if (cap > kPoolBlockBytes || dev->failed) {
@@ -189,24 +191,49 @@ static hipError_t release(fh_device *dev, uintptr_t base, size_t size) {
     while (drop < dev->pool.size() && (left > kPoolBytes || dev->pool.size() - drop >= kPoolBlocks))
         left -= dev->pool[drop++].capacity;
     hipError_t err = trim_pool(dev, drop);
-    dev->pool.push_back({base, cap});
+    dev->pool.push_back({base, cap, !ordered});
     dev->pool_bytes += cap;
     return err;
 }
 
-// The smallest kept block that serves `size`, or null.
-static void *take_pooled(fh_device *dev, size_t size) {
-    size_t best = dev->pool.size();
-    const size_t most = size + std::max<size_t>(size / 8, kPoolSlack);
-    for (size_t i = 0; i < dev->pool.size(); ++i) {
-        const size_t cap = dev->pool[i].capacity;
-        if (cap >= size && cap <= most && (best == dev->pool.size() || cap < dev->pool[best].capacity)) best = i;
+// *out: the smallest kept block that serves `size`, or null. Blocks that may
+// be in use on a caller's stream are left alone while the device's own stream
+// has work, until kSharedBlocks or kSharedBytes of them have gathered; then, as
+// hipFree does, the work queued on every stream of the GPU is waited for, once
+// for all of them. (14 ops of attention over 512 tokens, whose result the caller
+// reads: 276 us a pass, 304 with a wait at each such free.)
+static hipError_t take_pooled(fh_device *dev, size_t size, void **out) {
+    *out = nullptr;
+    const size_t none = dev->pool.size(), most = size + std::max<size_t>(size / 8, kPoolSlack);
+    size_t best = none, shared_blocks = 0;
+    uint64_t shared_bytes = 0;
+    bool shared_fits = false;
+    for (size_t i = 0; i < none; ++i) {
+        const PoolBlock &b = dev->pool[i];
+        const bool fits = b.capacity >= size && b.capacity <= most;
+        if (b.shared) {
+            ++shared_blocks;
+            shared_bytes += b.capacity;
+            shared_fits = shared_fits || fits;
+        } else if (fits && (best == none || b.capacity < dev->pool[best].capacity)) {
+            best = i;
+        }
     }
-    if (best == dev->pool.size()) return nullptr;
-    void *p = reinterpret_cast<void *>(dev->pool[best].base);
+    if (best == none) {
+        if (!shared_fits) return hipSuccess;
+        if (shared_blocks < kSharedBlocks && shared_bytes < kSharedBytes &&
+            hipStreamQuery(dev->stream) == hipErrorNotReady) {
+            (void)hipGetLastError();
+            return hipSuccess;
+        }
+        if (hipError_t err = hipDeviceSynchronize(); err != hipSuccess) return err;
+        for (PoolBlock &b : dev->pool) b.shared = false;
+        return take_pooled(dev, size, out);
+    }
+    *out = reinterpret_cast<void *>(dev->pool[best].base);
     dev->pool_bytes -= dev->pool[best].capacity;
     dev->pool.erase(dev->pool.begin() + static_cast<std::ptrdiff_t>(best));
-    return p;
+    return hipSuccess;
 }
 
 // Drops one graph's hold on each of its allocations; frees those the caller
@@ -222,15 +249,15 @@ static hipError_t drop_graph_refs(fh_device *dev, const fh_graph *g) {
         if (z == dev->retired.end()) continue;
         const size_t size = z->second;
         dev->retired.erase(z);
-        hipError_t err = release(dev, base, size);
+        hipError_t err = release(dev, base, size, false);
         if (first == hipSuccess) first = err;
     }
     return first;
 }
 
-// fh_free outside capture: a retained allocation is retired (no longer
-// usable by ops, freed with its last graph), any other one freed now.
-static int free_now(fh_device *dev, std::map<uintptr_t, size_t>::iterator it, const char *fn) {
+// A free outside capture: a retained allocation is retired (no longer
+// usable by ops, freed with its last graph), any other one released now.
+static int free_now(fh_device *dev, std::map<uintptr_t, size_t>::iterator it, const char *fn, bool ordered) {
     const uintptr_t base = it->first;
     const size_t size = it->second;
     dev->allocs.erase(it);
@@ -239,8 +266,8 @@ static int free_now(fh_device *dev, std::map<uintptr_t, size_t>::iterator it, co
         return FH_OK;
     }
     hipSetDevice(dev->ordinal);
-    hipError_t err = release(dev, base, size);
-    if (err != hipSuccess) return device_error(dev, err, fn, "hipStreamSynchronize/hipFree");
+    hipError_t err = release(dev, base, size, ordered);
+    if (err != hipSuccess) return device_error(dev, err, fn, "the wait for queued work or hipFree");
     return FH_OK;
 }
 
@@ -392,10 +419,11 @@ int fh_device_stream(fh_device *dev, void **stream) {
     return FH_OK;
 }
 
-// fh_alloc and fh_alloc_output. Work queued on the stream may still use a kept
-// block: unless `ordered` says that an op on that stream writes it first (or
-// the clearing below does), the caller may touch it from anywhere, so the
-// work is waited for, as fh_free did before it kept blocks.
+// fh_alloc and fh_alloc_output. Work queued on the device's stream may still
+// use a block that fh_free_ordered kept: unless `ordered` says that an op on
+// that stream writes it first (or the clearing below does), the caller may
+// touch it from anywhere, so that work is waited for. Work on other streams
+// has ended (take_pooled).
 static int allocate(fh_device *dev, size_t nbytes, int zero_fill, bool ordered, void **out, const char *fn) {
     if (!out) return fail(FH_ERR_INVALID_ARGUMENT, "%s: out is null", fn);
     *out = nullptr;
@@ -403,8 +431,9 @@ static int allocate(fh_device *dev, size_t nbytes, int zero_fill, bool ordered, 
     if (dev->capturing) return fail(FH_ERR_CAPTURE, "%s: cannot allocate while capturing", fn);
     if (int rc = set_current(dev, fn)) return rc;
     const size_t size = std::max<size_t>(nbytes, 1);
-    void *p = take_pooled(dev, size);
-    hipError_t err = hipSuccess;
+    void *p = nullptr;
+    hipError_t err = take_pooled(dev, size, &p);
+    if (err != hipSuccess) return device_error(dev, err, fn, "hipDeviceSynchronize");
     if (p != nullptr && !ordered && !zero_fill) {
         err = hipStreamSynchronize(dev->stream);
         if (err != hipSuccess) {
@@ -451,8 +480,8 @@ int fh_alloc_output(fh_device *dev, size_t nbytes, void **out) {
     return allocate(dev, nbytes, 0, true, out, "fh_alloc_output");
 }
 
-int fh_free(fh_device *dev, void *ptr) {
-    const char *fn = "fh_free";
+// fh_free and fh_free_ordered.
+static int free_allocation(fh_device *dev, void *ptr, bool ordered, const char *fn) {
     if (!dev) return fail(FH_ERR_INVALID_ARGUMENT, "%s: device is null", fn);
     if (!ptr) return FH_OK;
     auto it = dev->allocs.find(reinterpret_cast<uintptr_t>(ptr));
@@ -465,8 +494,12 @@ int fh_free(fh_device *dev, void *ptr) {
         dev->deferred_frees.push_back(ptr);
         return FH_OK;
     }
-    return free_now(dev, it, fn);
+    return free_now(dev, it, fn, ordered);
 }
+
+int fh_free(fh_device *dev, void *ptr) { return free_allocation(dev, ptr, false, "fh_free"); }
+
+int fh_free_ordered(fh_device *dev, void *ptr) { return free_allocation(dev, ptr, true, "fh_free_ordered"); }
 
 int fh_upload(fh_device *dev, void *dst, const void *src, size_t nbytes) {
     const char *fn = "fh_upload";
@@ -599,7 +632,7 @@ int run_deferred_frees(fh_device *dev, const char *fn) {
     for (void *p : pending) {
         auto it = dev->allocs.find(reinterpret_cast<uintptr_t>(p));
         if (it == dev->allocs.end()) continue;
-        const int r = free_now(dev, it, fn);
+        const int r = free_now(dev, it, fn, false);
         if (rc == FH_OK) rc = r;
     }
     return rc;

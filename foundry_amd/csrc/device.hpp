@@ -51,12 +51,17 @@ constexpr uint32_t kMaxGemmSplits = 8;
 constexpr uint64_t kPoolBytes = 512ull << 20;
 constexpr uint64_t kPoolBlockBytes = 128ull << 20;
 constexpr size_t kPoolBlocks = 256;
+// Of them, how many that may be in use on a caller's stream gather before
+// they are waited for (take_pooled).
+constexpr size_t kSharedBlocks = 16;
+constexpr uint64_t kSharedBytes = 16ull << 20;
 // A kept block serves a request it exceeds by at most this or 1/8 of it.
 constexpr uint64_t kPoolSlack = 64ull << 10;
 
 struct PoolBlock {
     uintptr_t base;
     size_t capacity;
+    bool shared;  // freed by fh_free: may be in use on a caller's stream
 };
 }  // namespace fh
 
@@ -69,11 +74,11 @@ struct fh_device {
     void *partial_area = nullptr;  // kPartialAreaBytes, likewise
     // base address -> size of every live allocation this device made
     std::map<uintptr_t, size_t> allocs;
-    // Freed blocks kept for reuse, oldest first, and their bytes. All work on
-    // a block is on the device's one stream, so whatever still uses it when
-    // it is freed runs before anything the next owner enqueues. capacity:
-    // bytes behind every block the device holds, live, retired or kept (a
-    // reused block may exceed the size asked for).
+    // Freed blocks kept for reuse, oldest first, and their bytes. What still
+    // uses one that is not shared is on the device's stream, so it runs before
+    // anything the next owner enqueues there.
+    // capacity: bytes behind every block the device holds, live, retired or
+    // kept (a reused block may exceed the size asked for).
     std::vector<fh::PoolBlock> pool;
     uint64_t pool_bytes = 0;
     std::unordered_map<uintptr_t, size_t> capacity;

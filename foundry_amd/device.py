@@ -23,22 +23,34 @@ from .primitive import (Binary, Cat, Copy, DType, IndexSelect, Matmul, Quantized
 
 class HipStorage:
     """One device allocation. Freed when the last reference drops, as the
-    reference's Rc<Storage> is (src/nn/tensor.rs:49-53)."""
+    reference's Rc<Storage> is (src/nn/tensor.rs:49-53).
 
-    __slots__ = ("device", "ptr", "nbytes", "views", "__weakref__")
+    ``ptr`` hands the address to the caller, who may use it on a stream of its
+    own: the memory then goes out again after the work queued on every stream
+    of the GPU. Storage whose address stayed inside HipDevice is freed in the
+    order of the device's stream."""
+
+    __slots__ = ("device", "_ptr", "_exported", "nbytes", "views", "__weakref__")
 
     def __init__(self, device: "HipDevice", ptr: int, nbytes: int):
         self.device = device
-        self.ptr = ptr
+        self._ptr = ptr
+        self._exported = False
         self.nbytes = nbytes
         self.views = 0  # live Tensor views (Rc::get_mut's uniqueness test)
 
+    @property
+    def ptr(self) -> int:
+        self._exported = True
+        return self._ptr
+
     def __del__(self):
         dev = self.device
-        if dev is not None and dev._handle and self.ptr:
+        if dev is not None and dev._handle and self._ptr:
             lib = _lib.load()
-            rc = lib.fh_free(dev._handle, ctypes.c_void_p(self.ptr))
-            self.ptr = 0
+            free = lib.fh_free if self._exported else lib.fh_free_ordered
+            rc = free(dev._handle, ctypes.c_void_p(self._ptr))
+            self._ptr = 0
             if rc != _lib.OK:
                 # a destructor cannot raise: report the lost allocation
                 warnings.warn(f"fh_free failed ({_lib.STATUS_NAMES.get(rc, rc)}): "
@@ -135,6 +147,10 @@ class Operand:
     def address(self) -> int:
         return self.storage.ptr + self.layout.offset * self.dtype.itemsize
 
+    def _address(self) -> int:
+        """The address for this module's own calls on the device's stream."""
+        return self.storage._ptr + self.layout.offset * self.dtype.itemsize
+
 
 class HipDevice:
     """One GPU, one HIP stream."""
@@ -216,7 +232,7 @@ class HipDevice:
         buf = np.ascontiguousarray(np.frombuffer(memoryview(data).cast("B"), dtype=np.uint8))
         st = self._alloc(buf.nbytes, zero=False)
         if buf.nbytes:
-            _lib.call("fh_upload", self.handle, ctypes.c_void_p(st.ptr),
+            _lib.call("fh_upload", self.handle, ctypes.c_void_p(st._ptr),
                       buf.ctypes.data_as(ctypes.c_void_p), buf.nbytes)
         return st
 
@@ -240,7 +256,7 @@ class HipDevice:
         out = np.empty(nbytes, dtype=np.uint8)
         if nbytes:
             _lib.call("fh_download", self.handle, out.ctypes.data_as(ctypes.c_void_p),
-                      ctypes.c_void_p(operand.address()), nbytes)
+                      ctypes.c_void_p(operand._address()), nbytes)
         return out.tobytes()
 
     def _owns(self, operand: Operand) -> None:
@@ -266,19 +282,19 @@ class HipDevice:
             rows, k = x.layout.shape
             if x.dtype is not DType.BF16:
                 raise _lib.HipError(_lib.ERR_DTYPE, "the q4 kernels take bf16 activations")
-            x_ptr, x_ld = x.address(), x.layout.strides[0] if rows > 1 else max(k, x.layout.strides[0])
+            x_ptr, x_ld = x._address(), x.layout.strides[0] if rows > 1 else max(k, x.layout.strides[0])
             if (k > 1 and x.layout.strides[1] != 1) or (rows > 1 and x.layout.strides[0] < k):
                 # The operand rule of the reference's matmul (matmul_operand,
                 # src/metal/mod.rs:384-401): rows the kernel cannot read in
                 # place (a column stride, overlapping or broadcast rows) are
                 # copied to a contiguous [rows, k] first.
                 staged = self._output(rows * k * 2)
-                _lib.call("fh_copy_strided", self.handle, int(x.dtype), ctypes.c_void_p(x.storage.ptr),
-                          ctypes.byref(x.layout.view()), ctypes.c_void_p(staged.ptr))
-                x_ptr, x_ld = staged.ptr, k
+                _lib.call("fh_copy_strided", self.handle, int(x.dtype), ctypes.c_void_p(x.storage._ptr),
+                          ctypes.byref(x.layout.view()), ctypes.c_void_p(staged._ptr))
+                x_ptr, x_ld = staged._ptr, k
             _lib.call("fh_q4_matmul", self.handle, ctypes.c_void_p(x_ptr), rows, k, x_ld,
-                      ctypes.c_void_p(wq.address()), ctypes.c_void_p(s.address()),
-                      ctypes.c_void_p(b.address()), shape[1], op.group, ctypes.c_void_p(out.ptr),
+                      ctypes.c_void_p(wq._address()), ctypes.c_void_p(s._address()),
+                      ctypes.c_void_p(b._address()), shape[1], op.group, ctypes.c_void_p(out._ptr),
                       _lib.BF16 if out_dtype is DType.BF16 else _lib.F32)
             return out
         if isinstance(op, QuantizedIndexSelect):
@@ -287,9 +303,9 @@ class HipDevice:
                 if not w.layout.is_contiguous():
                     raise TensorError("IndexSelectIncompatible", "operands must be contiguous")
             rows = wq.layout.shape[0]
-            _lib.call("fh_q4_embed", self.handle, ctypes.c_void_p(wq.address()),
-                      ctypes.c_void_p(s.address()), ctypes.c_void_p(b.address()), rows, shape[1],
-                      op.group, ctypes.c_void_p(ids.address()), shape[0], ctypes.c_void_p(out.ptr))
+            _lib.call("fh_q4_embed", self.handle, ctypes.c_void_p(wq._address()),
+                      ctypes.c_void_p(s._address()), ctypes.c_void_p(b._address()), rows, shape[1],
+                      op.group, ctypes.c_void_p(ids._address()), shape[0], ctypes.c_void_p(out._ptr))
             return out
         self._run_standard(op, inputs, shape, out_dtype, out)
         return out
@@ -297,10 +313,10 @@ class HipDevice:
     def _run_standard(self, op, inputs, shape, dtype, out) -> None:
         """The reference's own Ops through the strided entry points
         (MetalDevice::run, src/metal/mod.rs:639-695)."""
-        h, dst = self.handle, out.ptr
+        h, dst = self.handle, out._ptr
 
         def base(o):
-            return o.storage.ptr
+            return o.storage._ptr
 
         def view(o):
             return ctypes.byref(o.layout.view())
@@ -341,8 +357,8 @@ class HipDevice:
         (src,) = inputs
         self._owns(src)
         _lib.call("fh_slice_scatter", self.handle, int(target.dtype), op.dim, op.start,
-                  ctypes.c_void_p(target.storage.ptr), ctypes.byref(target.layout.view()),
-                  ctypes.c_void_p(src.storage.ptr), ctypes.byref(src.layout.view()))
+                  ctypes.c_void_p(target.storage._ptr), ctypes.byref(target.layout.view()),
+                  ctypes.c_void_p(src.storage._ptr), ctypes.byref(src.layout.view()))
 
     # ---- batching and timing (CommandStream counterpart) ----
     def capture_begin(self) -> None:

@@ -216,7 +216,7 @@ def test_time() -> str:
 class _CallTimer:
     """Brackets every C-ABI compute call with device events while active."""
 
-    SKIP = {"fh_upload", "fh_download", "fh_alloc", "fh_alloc_output", "fh_free", "fh_synchronize", "fh_timer_begin",
+    SKIP = {"fh_upload", "fh_download", "fh_alloc", "fh_alloc_output", "fh_free", "fh_free_ordered", "fh_synchronize", "fh_timer_begin",
             "fh_timer_end", "fh_take_profile", "fh_device_stream"}
 
     def __init__(self, dev):

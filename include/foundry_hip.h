@@ -111,20 +111,24 @@ int fh_device_stream(fh_device *dev, void **stream);
 int fh_alloc(fh_device *dev, size_t nbytes, int zero_fill, void **out);
 /* The same without the clearing, for storage that an op on the device's
  * stream writes before anything else touches it (an op's output): a block
- * kept by fh_free is handed out without a wait for the work queued on it. */
+ * kept for reuse is handed out without a wait for the work queued on it. */
 int fh_alloc_output(fh_device *dev, size_t nbytes, void **out);
-/* Frees an allocation of this device. Work already queued on the device's
- * stream may still use the memory; it is then kept for later fh_alloc calls
- * of the device (at most 512 MiB, blocks of at most 128 MiB, the oldest given
- * back first, all of them when the driver runs out) or given back to the
- * driver once that work ends. Memory in use on a stream of the caller's own
- * must not be freed before that use ends.
+/* Frees an allocation of this device. The memory is given back to the driver,
+ * or kept for later allocations of the device (at most 512 MiB, blocks of at
+ * most 128 MiB, the oldest given back first, all of them when the driver runs
+ * out), after the work queued on the GPU, on any stream, ends: the call itself
+ * may return before.
  * A live graph retains every allocation its captured ops touched, as a
  * Metal command buffer retains its buffers (src/metal/mod.rs:280-282): the
  * allocation is then no longer usable by ops but stays allocated until the
  * last graph that uses it is destroyed. A free asked for while capturing is
  * carried out at fh_capture_end, on the same rule. */
 int fh_free(fh_device *dev, void *ptr);
+/* The same for memory that only ops on the device's stream (and fh_upload,
+ * fh_download) have touched, such as an op's output that never left the
+ * device: no other stream is waited for, since queued work that still uses it
+ * runs before anything that a later owner enqueues. */
+int fh_free_ordered(fh_device *dev, void *ptr);
 /* Host -> device copy into an owned range; ordered on the stream. */
 int fh_upload(fh_device *dev, void *dst, const void *src, size_t nbytes);
 /* Device -> host copy of an owned range; synchronises first. */
@@ -134,7 +138,7 @@ int fh_download(fh_device *dev, void *dst, const void *src, size_t nbytes);
  * Bytes counted: every live allocation (including retired ones a graph still
  * holds) plus the device's own work areas (the 33 MB of GEMV/GEMM partial
  * sums and the batched GEMV's x image), allocated at creation; freed blocks
- * kept for reuse (fh_free) are not counted. */
+ * kept for reuse (fh_free, at most 512 MiB) are not counted. */
 int fh_max_memory_allocated(const fh_device *dev, fh_allocated_memory *out);
 int fh_reset_run_memory_peak(fh_device *dev);
 int fh_run_memory_peak(const fh_device *dev, fh_allocated_memory *out);

@@ -552,33 +552,81 @@ def test_freed_blocks_are_reused_in_stream_order(nbytes):
         dev.close()
 
 
+def _stream_query(dev):
+    """hipStreamQuery (found through the library's own dependency), and the
+    device's stream."""
+    ptr = ctypes.c_void_p()
+    _lib.call("fh_device_stream", dev.handle, ctypes.byref(ptr))
+    query = _lib.load().hipStreamQuery
+    query.argtypes = [ctypes.c_void_p]
+    return query, ptr
+
+
 @pytest.mark.parametrize("kept", [True, False])
 def test_fresh_storage_is_idle_on_return(kept):
     """Storage from empty() may be written from any stream at once: the queued
     work that still uses a kept block has ended by then. Op outputs are not
-    waited for (the op writes them in stream order) and hold the op's result."""
+    waited for (the op writes them in stream order) and hold the op's result;
+    nor does an allocation that no kept block serves disturb the queued work."""
     dev = HipDevice(0)
     try:
-        ptr = ctypes.c_void_p()
-        _lib.call("fh_device_stream", dev.handle, ctypes.byref(ptr))
-        query = _lib.load().hipStreamQuery  # found through the library's own dependency
-        query.argtypes = [ctypes.c_void_p]
-        n = 1024
+        query, stream = _stream_query(dev)
+        n = 2048
         an = np.random.default_rng(7).standard_normal((n, n)).astype(np.float32)
         a = f32(dev, an, an.shape)
-        dev.synchronize()
-        out = None
-        for _ in range(40):
-            out = a.matmul(dev, a)
-        want = out.to_numpy(dev)
-        for _ in range(40):
+        want = a.matmul(dev, a).to_numpy(dev)
+        for _ in range(60):  # about 0.3 ms each, issued in a tenth of that
             out = a.matmul(dev, a)
         nbytes = n * n * 4
+        assert query(stream) != 0, "the queued work ended before it could be waited for"
         del out  # its kernel is still queued
+        assert query(stream) != 0, "freeing an op's output waits"
         fresh = dev.empty(nbytes if kept else 2 * nbytes)
         if kept:
-            assert query(ptr) == 0
+            assert query(stream) == 0
         del fresh
         assert np.array_equal(a.matmul(dev, a).to_numpy(dev), want)
     finally:
+        dev.close()
+
+
+def test_freed_memory_waits_for_the_callers_streams():
+    """Memory whose address was handed out may be in use on a stream of the
+    caller's own when it is freed: it goes to its next owner only after that. An
+    op's output that never left the device goes out again without such a
+    wait."""
+    dev = HipDevice(0)
+    lib = _lib.load()
+    own = ctypes.c_void_p()
+    lib.hipMemcpyAsync.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_int, ctypes.c_void_p]
+    lib.hipStreamDestroy.argtypes = [ctypes.c_void_p]
+    assert lib.hipStreamCreateWithFlags(ctypes.byref(own), ctypes.c_uint(1)) == 0  # hipStreamNonBlocking
+    try:
+        query, _ = _stream_query(dev)
+        n = 64 << 20
+        ones = f32(dev, np.ones(n // 4, np.float32), (n // 4,))
+        srcs, dst = [dev.zeros(n) for _ in range(3)], dev.empty(n)
+        old = {src.ptr for src in srcs}
+        dev.synchronize()
+
+        def read_sources():
+            for _ in range(150):  # about 30 us each, device to device
+                for src in srcs:
+                    assert lib.hipMemcpyAsync(dst.ptr, src.ptr, n, 3, own) == 0
+            assert query(own) != 0, "the copies ended before the free"
+
+        read_sources()
+        for _ in range(20):
+            ones.add(dev, ones)
+        assert query(own) != 0, "an op's output waits for other streams"
+        read_sources()
+        del srcs  # more than the blocks that gather before they are waited for
+        twos = [ones.add(dev, ones) for _ in range(4)]
+        assert old & {t.storage.ptr for t in twos}, "no block went out again"
+        dev.synchronize()
+        host = np.ones(n, np.uint8)
+        _lib.call("fh_download", dev.handle, host.ctypes.data_as(ctypes.c_void_p), dst.ptr, n)
+        assert not host.any()
+    finally:
+        lib.hipStreamDestroy(own)
         dev.close()

@@ -126,7 +126,7 @@ def test_draw_inputs_order_and_golden_prompt():
     assert s3.shape == (2,)
 
 
-@pytest.mark.parametrize("name", ["fh_alloc", "fh_alloc_output", "fh_free"])
+@pytest.mark.parametrize("name", ["fh_alloc", "fh_alloc_output", "fh_free", "fh_free_ordered"])
 def test_call_timer_counts_no_allocation(monkeypatch, name):
     """Allocating and freeing storage are no dispatches of a step's profile."""
     seen = []
