@@ -14,6 +14,7 @@
 #include <utility>
 
 #include "device.hpp"
+#include "q4_gemm.hpp"
 
 namespace fh {
 int check_q4_table(const fh_device *dev, const char *fn, const uint32_t *wq, const uint16_t *scales,
@@ -26,9 +27,6 @@ void launch_rms_norm_partials(hipStream_t stream, const float *part, uint32_t sp
                               uint16_t *y);
 void launch_silu_mul_partials(hipStream_t stream, const float *part, uint32_t splits, uint32_t rows, uint32_t f,
                               uint16_t *out);
-bool launch_q4_gemm_direct_silu(hipStream_t stream, uint32_t cus, const uint16_t *x, uint32_t x_ld,
-                                const uint32_t *wq, const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t f,
-                                uint32_t k, uint16_t *act);
 bool attention_flash_applies(uint32_t cus, uint32_t rows, uint32_t n_heads, uint32_t n_kv, uint32_t head_dim,
                              uint32_t max_len, float scale);
 bool launch_attention_flash(hipStream_t stream, uint32_t cus, const uint16_t *q, const uint32_t *positions,
@@ -206,8 +204,9 @@ int add_norm(fh_device *d, const fh_llama_model &m, int64_t rows, const uint16_t
 }
 
 // Above 8 rows: gate_up = m.x [Wgate; Wup]^T; act = silu(gate) * up, in the
-// GEMM's epilogue where its tiles fill the chip, else the SiLU forming gate
-// and up from the GEMM's output or split partials (linear_deferred).
+// GEMM's epilogue where it is the direct one and its tiles fill the chip, else
+// the SiLU forming gate and up from the GEMM's output or split partials
+// (linear_deferred).
 int linear_silu(fh_device *d, const fh_llama_model &m, int64_t rows, const fh_q4_weight &w) {
     const char *fn = "fh_llama_forward";
     if (m.ffn % 8 != 0 || !aligned16(m.act)) {
@@ -220,13 +219,13 @@ int linear_silu(fh_device *d, const fh_llama_model &m, int64_t rows, const fh_q4
     FH_TRY(fh::check_range(d, m.act, static_cast<uint64_t>(rows) * m.ffn * 2, fn, "act"));
     // prompt-length rows whose tiles fill the chip: the activation in the
     // GEMM's epilogue (no gate/up tensor, no SiLU launch)
-    bool fused = false;
-    FH_TRY(fh::dispatch(d, fn, [&] {
-        fused = fh::launch_q4_gemm_direct_silu(d->stream, d->compute_units, m.x, static_cast<uint32_t>(m.hidden), w.wq,
-                                               w.scales, w.biases, static_cast<uint32_t>(rows),
-                                               static_cast<uint32_t>(m.ffn), static_cast<uint32_t>(m.hidden), m.act);
-    }));
-    if (fused) return FH_OK;
+    const uint32_t mm = static_cast<uint32_t>(rows), f = static_cast<uint32_t>(m.ffn);
+    const uint32_t k = static_cast<uint32_t>(m.hidden);
+    if (fh::direct_silu_applies(d->compute_units, k, mm, f, k, m.act) &&
+        fh::q4_gemm_rows_plan(d->compute_units, k, w.scales, w.biases, mm, 2 * f, k, true).ct == 0)
+        return fh::dispatch(d, fn, [&] {
+            fh::launch_q4_gemm_direct_silu(d->stream, m.x, k, w.wq, w.scales, w.biases, mm, f, k, m.act);
+        });
     uint32_t splits = 1;
     FH_TRY(gemm_deferred(d, fn, m.x, rows, m.hidden, w, m.gate_up, &splits));
     if (splits == 1) return fh_silu_mul(d, m.gate_up, rows, m.ffn, m.act);

@@ -342,6 +342,15 @@ static double tiled_gemm_us(uint32_t cus, uint32_t x_ld, uint32_t m, uint32_t n,
 // - weights straight to the matrix cores (q4_gemm_direct.hip) where its
 //   256 x 256 tiles fill the chip, or 3/4 of it over two K ranges;
 // - q4_gemm_kernel otherwise.
+// The same rule serves the [gate; up] GEMM with its activation (bit for bit the
+// plain GEMM and fh_silu_mul): q4_gemm_rows_plan says when it is the first.
+RowsPlan q4_gemm_rows_plan(uint32_t cus, uint32_t x_ld, const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t n,
+                           uint32_t k, bool area) {
+    const RowsPlan rows = plan_q4_gemm_rows(cus, x_ld, s, b, m, n, k);
+    if (rows.ct != 0 && rows.us * (m < 512 ? 1.03 : 1.43) < tiled_gemm_us(cus, x_ld, m, n, k, area)) return rows;
+    return RowsPlan();
+}
+
 // launch_q4_gemm_deferred leaves a K split's f32 partials in `area`
 // (kPartialAreaBytes) and returns the split count (1: y was written), so that
 // a consumer of y can add the partials itself, in the order
@@ -349,8 +358,8 @@ static double tiled_gemm_us(uint32_t cus, uint32_t x_ld, uint32_t m, uint32_t n,
 uint32_t launch_q4_gemm_deferred(hipStream_t stream, uint32_t cus, const uint16_t *x, uint32_t x_ld,
                                  const uint32_t *wq, const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t n,
                                  uint32_t k, void *y, int y_is_f32, void *area) {
-    const RowsPlan rows = plan_q4_gemm_rows(cus, x_ld, s, b, m, n, k);
-    if (rows.ct != 0 && rows.us * (m < 512 ? 1.03 : 1.43) < tiled_gemm_us(cus, x_ld, m, n, k, area != nullptr)) {
+    const RowsPlan rows = q4_gemm_rows_plan(cus, x_ld, s, b, m, n, k, area != nullptr);
+    if (rows.ct != 0) {
         launch_q4_gemm_rows(stream, rows, x, x_ld, wq, s, b, m, n, k, y, y_is_f32);
         return 1;
     }

@@ -562,25 +562,28 @@ uint32_t launch_q4_gemm_direct(hipStream_t stream, uint32_t cus, const uint16_t 
 }
 
 // act [m][f] = silu_mul1 of the [gate; up] GEMM (n = 2 f weight rows) in one
-// launch (y_mode 3), when its 256-row x 128-pair tiles fill the chip with no
+// launch (y_mode 3): where its 256-row x 128-pair tiles fill the chip with no
 // K split, f % 128 == 0, k % 512 == 0, act 16-byte aligned and every byte
-// offset within 32 bits. Returns false when it does not apply.
-bool launch_q4_gemm_direct_silu(hipStream_t stream, uint32_t cus, const uint16_t *x, uint32_t x_ld,
-                                const uint32_t *wq, const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t f,
-                                uint32_t k, uint16_t *act) {
+// offset within 32 bits.
+bool direct_silu_applies(uint32_t cus, uint32_t x_ld, uint32_t m, uint32_t f, uint32_t k, const uint16_t *act) {
     const uint32_t n = 2 * f;
-    const uint32_t tiles_m = (m + kDBM - 1) / kDBM, tiles_n = f / (kDBN / 2);
-    const uint64_t tiles = static_cast<uint64_t>(tiles_m) * tiles_n;
+    const uint64_t tiles = static_cast<uint64_t>((m + kDBM - 1) / kDBM) * (f / (kDBN / 2));
     if (f == 0 || f % (kDBN / 2) != 0 || m == 0 || tiles < cus || tiles > 0x7FFFFFFFull || k == 0 ||
         k % (kDSbGroups * kDBK) != 0 || (reinterpret_cast<uintptr_t>(act) & 15) != 0)
         return false;
-    if (static_cast<uint64_t>(m) * x_ld * 2 >= (1ull << 32) || static_cast<uint64_t>(n) * k / 2 >= (1ull << 32))
-        return false;
+    return static_cast<uint64_t>(m) * x_ld * 2 < (1ull << 32) && static_cast<uint64_t>(n) * k / 2 < (1ull << 32);
+}
+
+void launch_q4_gemm_direct_silu(hipStream_t stream, const uint16_t *x, uint32_t x_ld, const uint32_t *wq,
+                                const uint16_t *s, const uint16_t *b, uint32_t m, uint32_t f, uint32_t k,
+                                uint16_t *act) {
+    const uint32_t n = 2 * f;
+    const uint32_t tiles_m = (m + kDBM - 1) / kDBM, tiles_n = f / (kDBN / 2);
+    const uint64_t tiles = static_cast<uint64_t>(tiles_m) * tiles_n;
     direct_lds_opt_in();
     const uint32_t gm = xcd_rect_rows(tiles, tiles_m, tiles_n, k);  // a tile reads 256 weight rows either way
     hipLaunchKernelGGL(q4_gemm_direct_kernel, dim3(static_cast<uint32_t>(tiles)), dim3(kDThreads), kDLds, stream, x,
                        x_ld, wq, s, b, m, n, k, act, 3, tiles_m, tiles_n, gm, k);
-    return true;
 }
 
 }  // namespace fh

@@ -419,8 +419,9 @@ int fh_decode_attention_noalloc(fh_device *dev, const uint16_t *qkv, int64_t bat
  *     [m, f] bf16. x' = x, or with norm_weight, the RMSNorm above (residual
  *     arguments as for fh_q4_matmul_rmsnorm). Above 8 rows, without a norm
  *     weight or residual: the prompt GEMM with the activation in its
- *     epilogue, when its tiles of 256 rows x 128 gate/up pairs fill the GPU
- *     (f % 128 == 0, k % 512 == 0; x and act 16-byte aligned, act not
+ *     epilogue (few rows: the GEMM, its sums in the device's partial area, and
+ *     the activation), when its tiles of 256 rows x 128 gate/up pairs fill the
+ *     GPU (f % 128 == 0, k % 512 == 0; x and act 16-byte aligned, act not
  *     overlapping x); other shapes return FH_ERR_UNSUPPORTED. Bit-identical
  *     to fh_q4_matmul then fh_silu_mul.
  * The q4 operands follow fh_q4_matmul (group 64); x 16-byte aligned. */

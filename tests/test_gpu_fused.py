@@ -151,6 +151,26 @@ def test_gate_up_silu_prompt_rows(device, m, k, f):
     assert np.count_nonzero(got) > got.size // 2  # a real activation, not a cleared buffer
 
 
+# Rows that fh_q4_matmul gives to the few-row kernel, 1, 2 and 4 row tiles;
+# the last one's sums are more than the 128 MiB area they pass through holds
+# (63 of the 64 rows at a time)
+@pytest.mark.parametrize("m,k,f", [(16, 512, 32768), (24, 1024, 40960), (64, 1024, 40960), (64, 1536, 266240)])
+def test_gate_up_silu_few_rows(device, m, k, f):
+    """The activation of few rows over a wide [gate; up] is bit-identical to
+    fh_q4_matmul followed by fh_silu_mul, which take the few-row kernel there."""
+    (wq, s, b), _ = q4(device, 95 + m, 1024, k)
+    w = [up(device, np.tile(a, (2 * f // 1024, 1))) for a in (wq, s, b)]
+    sx, act = up(device, synth.bf16_normal(96 + m, (m, k))), device.empty(m * f * 2)
+    _lib.call("fh_q4_gate_up_silu", device.handle, P(sx), None, None, None, ctypes.c_float(EPS), m, k, P(w[0]),
+              P(w[1]), P(w[2]), 2 * f, 64, P(act))
+    gu, want = device.empty(m * 2 * f * 2), device.empty(m * f * 2)
+    _lib.call("fh_q4_matmul", device.handle, P(sx), m, k, k, P(w[0]), P(w[1]), P(w[2]), 2 * f, 64, P(gu), _lib.BF16)
+    _lib.call("fh_silu_mul", device.handle, P(gu), m, f, P(want))
+    got, want = down(device, act, np.uint16, m * f), down(device, want, np.uint16, m * f)
+    assert np.array_equal(got, want), np.count_nonzero(got != want)
+    assert np.count_nonzero(got) > got.size // 2
+
+
 @pytest.mark.parametrize("m", [1, 3])
 def test_gate_up_silu_with_rmsnorm(device, m):
     """Norm prologue and SiLU epilogue together equal fh_q4_matmul_rmsnorm's
