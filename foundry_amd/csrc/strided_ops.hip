@@ -4,12 +4,12 @@
 // conversion, unary and binary elementwise ops, row reductions, matmul,
 // index_select, cat and slice_scatter, each over strided views.
 //
-// These are plain kernels, one output element per thread (one block per
-// output element for the reductions; the matmul on the fp32 matrix cores),
-// with the Metal kernels' arithmetic:
-// values decoded to fp32, the op in fp32, one rounding on the way out
-// (src/metal/kernels/common.metal:29-43). They serve the model code that
-// runs op by op; the decoder's hot path has its own fused kernels.
+// Elementwise ops and moves take 16-byte pieces where the views allow it and
+// single elements otherwise; reductions run a block or a wavefront per output
+// element; the matmul runs on the fp32 matrix cores. All with the Metal
+// kernels' arithmetic: values decoded to fp32, the op in fp32, one rounding on
+// the way out (src/metal/kernels/common.metal:29-43). They serve the model code
+// that runs op by op; the decoder's hot path has its own fused kernels.
 #include <type_traits>
 
 #include "device.hpp"
@@ -333,19 +333,20 @@ __global__ __launch_bounds__(kThreads) void argmax_kernel(const typename Float<D
 // Batched matmul over strided operands on the matrix cores, in fp32:
 // v_mfma_f32_16x16x4_f32 adds its four products to the accumulator one fma at
 // a time in order of k, so every sum is the chain of fmas over k that
-// matmul_tiled forms (src/metal/kernels/matmul.metal:42-64); checked bit for
-// bit on the GPU against fmaf for 1M sums of normal, huge, tiny, denormal,
-// infinite and NaN values.
+// matmul_tiled forms (src/metal/kernels/matmul.metal:42-64), also for huge,
+// tiny, denormal, infinite and NaN values.
 // A block of four wavefronts (WM x WN) owns WM * 16 T rows x WN * 16 T columns
 // of one batch entry; operand tiles of 32 along k go through LDS as fp32, the
 // next tile's global loads in flight while one is computed. In LDS a row's (or
 // column's) 32 values lie by k % 4, then k / 4, 8 together: a lane's operands
 // of 8 MFMAs are two conflict-free 16-byte reads. Values past k are filled
 // with +0 (lhs) and -0 (rhs), whose product leaves every sum as it is.
-// Bounded by the fp32 matrix-core rate (157 TFLOP/s). Before, a thread kept
-// 2 x 2 sums fed by scalar LDS reads. bf16, before and now: 24 x [512, 128] x
-// [128, 512] (keys transposed in place) 69.2 -> 26.5 us, 24 x [512, 512] x
-// [512, 128] 73.9 -> 34.2 us, [16, 3072] x [3072, 8192] 224.6 -> 74.4 us.
+// Before, a thread kept 2 x 2 sums fed by scalar LDS reads. bf16, before and
+// now: 24 x [512, 128] x [128, 512] (keys transposed in place) 69.2 -> 26.5 us
+// (61 TFLOP/s, 0.39 of the fp32 matrix-core rate), 24 x [512, 512] x [512, 128]
+// 73.9 -> 34.2 us, [16, 3072] x [3072, 8192] 224.6 -> 74.4 us. Neither that rate
+// nor memory bounds it but the chain of steps: two barriers around one LDS
+// buffer per 32 of k (the last shape: 96 steps of 0.78 us in a block per CU).
 struct MatmulShape {
     uint32_t m, n, k, batch_ndim;
     uint32_t batch_dims[2];
@@ -868,8 +869,15 @@ extern "C" int fh_reduce(fh_device *dev, int op, int dtype, const void *src, con
     const int64_t stride = view->strides[dim];
     const uint32_t size = static_cast<uint32_t>(dim_size);
     // A wavefront per row where the rows alone give every CU 4 blocks of
-    // them, else a block per row.
-    if (op != FH_ARGMAX && rows >= 16ll * dev->compute_units) {
+    // them, else a block per row. Sums of 4096 rows, block / wavefront per row:
+    // f32 512 long 5.9 / 3.7 us, 8192 27.9 / 20.7, 128256 583 / 363; bf16 512
+    // 5.9 / 3.9, 128256 530 / 294. Along a strided dim also (8192 rows of 64 f32
+    // 8.6 / 4.1, of 4096 225 / 178), except f32 rows of 256 to 2047 values while
+    // there are fewer than 256 rows a CU: 4096 of 512 12.5 / 14.2, 8192 of 1024
+    // 38.9 / 47.3 (65536 of 256 81.2 / 79.3).
+    const bool block_strided = dtype == FH_F32 && stride > 1 && size >= 256 && size < 2048 &&
+                               rows < 256ll * dev->compute_units;
+    if (op != FH_ARGMAX && rows >= 16ll * dev->compute_units && !block_strided) {
         return dispatch(dev, fn, [&] {
             const uint32_t n_rows = static_cast<uint32_t>(rows);
             const uint32_t blocks = n_rows / 4 + 1;

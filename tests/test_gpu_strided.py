@@ -431,11 +431,11 @@ def test_elementwise_and_moves_over_every_walk(device, dtype, shape):
 
 
 @pytest.mark.parametrize("dtype", [DType.F32, DType.BF16])
-@pytest.mark.parametrize("size", [1, 63, 64, 65, 192, 255, 256, 257, 700])
+@pytest.mark.parametrize("size", [1, 63, 64, 65, 192, 255, 256, 257, 700, 2047, 2048])
 def test_reductions_of_many_rows(device, dtype, size):
-    """At least 16 rows per CU are reduced a wavefront per row, in the order of
-    the 256-thread fold and tree all the same; along the last dim and a
-    strided one."""
+    """At least 16 rows per CU are reduced a wavefront per row (f32 rows of 256
+    to 2047 along a strided dim a block), in the order of the 256-thread fold
+    and tree all the same; along the last dim and a strided one."""
     rng = np.random.default_rng(size)
     an = _as_dtype(rng.standard_normal((8200, size)).astype(np.float32), dtype)
     for t, dim in ((f32(device, an, an.shape), 1), (f32(device, an.T, an.T.shape), 0)):
