@@ -487,6 +487,68 @@ def test_matmul_sums_are_the_chain_over_k(device, dtype, batch, m, k, n):
         assert np.array_equal(got.view(exact.dtype), exact), (lhow, rhow)
 
 
+SPECIALS = np.array([np.inf, -np.inf, np.nan, 0.0, -0.0, 3.0e38, -3.0e38, 1.0e-40, -1.0e-40, 1.0e-30], np.float32)
+
+
+@pytest.mark.parametrize("dtype", [DType.F32, DType.BF16])
+@pytest.mark.parametrize("rows,size", [(40, 1), (40, 300), (8200, 1), (8200, 65), (8200, 300)])
+def test_reductions_of_special_values(device, dtype, rows, size):
+    """Sums and maxima over infinities, NaNs and values at the ends of the
+    range, a block and a wavefront per row: sums in the restated order; a
+    maximum leaves NaNs out (fmax), and is -inf where there is nothing else."""
+    rng = np.random.default_rng(rows + size)
+    an = _as_dtype(rng.standard_normal((rows, size)).astype(np.float32), dtype)
+    an[::3, rng.integers(0, size, 2)] = _as_dtype(rng.choice(SPECIALS, (len(an[::3]), 2)), dtype)
+    an[1] = np.nan
+    an[2] = -np.inf
+    for t, dim in ((f32(device, an, an.shape), 1), (f32(device, an.T, an.T.shape), 0)):
+        t = t.to_dtype(device, dtype)
+        s, m = values(device, t.sum_keepdim(device, dim)), values(device, t.amax_keepdim(device, dim))
+        with np.errstate(invalid="ignore", over="ignore"):
+            want = _as_dtype(_reduce_restated(an, False), dtype)
+        assert np.array_equal(s.ravel(), want, equal_nan=True), dim
+        assert np.array_equal(m.ravel(), np.fmax.reduce(an, axis=1, initial=-np.inf)), dim
+
+
+@pytest.mark.parametrize("dim", [0, 1])
+def test_sum_of_an_empty_dim(device, dim):
+    """A sum over no element is 0, for few rows and many."""
+    for rows in (3, 8200):
+        t = Tensor.zeros(device, DType.F32, (rows, 0) if dim else (0, rows))
+        assert not t.sum_keepdim(device, dim).to_numpy(device).any()
+
+
+@pytest.mark.parametrize("transposed", [False, True])
+def test_matmul_chain_of_fmas(device, transposed):
+    """In F32 every sum is the chain of fused multiply-adds over k, bit for bit
+    against the C library's fmaf: full significands (a separate multiply and
+    add rounds otherwise), values at both ends of the range, denormals, zeros
+    of both signs, infinities and NaNs."""
+    fmaf = ctypes.CDLL("libm.so.6").fmaf
+    fmaf.restype, fmaf.argtypes = ctypes.c_float, [ctypes.c_float] * 3
+    rng = np.random.default_rng(17)
+    m, k, n = 21, 37, 19
+    kinds = [lambda s: rng.standard_normal(s), lambda s: rng.standard_normal(s) * 1e30,
+             lambda s: rng.standard_normal(s) * 1e-25, lambda s: rng.standard_normal(s) * 1e-41,
+             lambda s: rng.choice(SPECIALS, s)]
+    a = np.stack([kinds[i % 5](k) for i in range(m)]).astype(np.float32)
+    b = np.stack([kinds[j // 5 % 5](k) for j in range(n)], axis=1).astype(np.float32)
+    want = np.zeros((m, n), np.float32)
+    for i in range(m):
+        for j in range(n):
+            acc = 0.0
+            for kk in range(k):
+                acc = fmaf(float(a[i, kk]), float(b[kk, j]), acc)
+            want[i, j] = acc
+    lt = f32(device, a, a.shape)
+    rt = f32(device, b.T, (n, k)).permute((1, 0)) if transposed else f32(device, b, b.shape)
+    got = lt.matmul(device, rt).to_numpy(device)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and not np.isnan(want).all()
+    ok = ~np.isnan(want)
+    assert np.array_equal(got[ok].view(np.uint32), want[ok].view(np.uint32))
+    assert np.count_nonzero(np.isinf(want)) and np.count_nonzero((np.abs(want) < 1e-38) & (want != 0))
+
+
 def test_strided_entry_points_reject_bad_views(device):
     """Out-of-allocation views and mismatched dims are refused on the host."""
     import ctypes
