@@ -1406,11 +1406,14 @@ constexpr int kShortDims = FH_DECODE_SHORT_DIMS;  // V dims per block
 
 // Launches the one-launch kernel where its blocks, n_kv * HD / kShortDims per
 // row and a wavefront per chunk, run at once or nearly (up to a third of a
-// second round); false otherwise. In more rounds every block pulls its head's
+// second round, see below); false otherwise. In more rounds every block pulls its head's
 // keys through a CU again, which the split form does not: 8 rows of 8 KV heads
 // of 128, 1000 positions, 74.8 us against 15.7 us split; 2 rows at 768 16.3 /
 // 11.2; on the other side 2 rows at 500 9.8 / 11.1, one row at 1000 11.0 /
-// 11.1, and 8 rows of heads of 64 at 500 (a round and a third) 12.6 / 13.5.
+// 11.1, and 8 rows of heads of 64 at 500 (a round and a third) 12.6 / 13.5. With
+// heads of 64 and at most 256 positions two rounds pay too: 12 rows at 200 9.3 /
+// 12.6, 16 rows 11.0 / 12.6, 16 rows at 64 8.6 / 9.3 (24 rows, three rounds, 11.8
+// / 9.9; 16 rows at 400 18.4 / 14.0).
 template <int HD, int G>
 static bool launch_decode_short(hipStream_t stream, uint32_t cus, uint32_t rows, const AttnArgs &x) {
     // one wavefront per 64-key chunk the cache can hold (positions beyond
@@ -1434,7 +1437,8 @@ static bool launch_decode_short(hipStream_t stream, uint32_t cus, uint32_t rows,
         resident[waves].store(per_cu, std::memory_order_relaxed);
     }
     const dim3 grid(x.n_kv * (HD / kShortDims), rows);
-    if (3ull * grid.x * rows > 4ull * cus * static_cast<uint64_t>(per_cu)) return false;
+    const uint64_t blocks = static_cast<uint64_t>(grid.x) * rows, round = cus * static_cast<uint64_t>(per_cu);
+    if (3 * blocks > 4 * round && !(HD == 64 && x.max_len <= 256 && blocks <= 2 * round)) return false;
     hipLaunchKernelGGL((attn_decode_short_kernel<HD, G, kShortDims>), grid, dim3(64 * waves), 0, stream, x.q_src, x.cos_tab,
                        x.sin_tab, x.positions, x.pos_limit, x.k_cache, x.v_cache, x.row_stride, x.n_heads, x.n_kv,
                        x.max_len, x.scale, x.out);

@@ -429,9 +429,11 @@ def test_decode_attention(device, n_heads, n_kv, hd, batch, max_len):
 # Both sides of the rules that pick the decode form: caches of at most 1024
 # positions whose one-launch blocks run at once (8 rows of 8 heads of 128 at
 # 100, of 64 at 500) or would take more rounds (the same at 200 and 1000, 3
-# rows at 350, 32 KV heads at 1000), and the sliced or chunked P.V on either
-# side of 448 positions (head_dim 256 never takes the one-launch form).
-DECODE_RULE_CASES = [(32, 8, 128, 8, 100), (32, 8, 64, 8, 500), (32, 8, 128, 8, 200), (32, 8, 128, 8, 1000),
+# rows at 350, 32 KV heads at 1000), two rounds with heads of 64 up to 256
+# positions (16 rows at 256; not at 257, nor 17 rows), and the sliced or chunked
+# P.V on either side of 448 positions (head_dim 256 never takes the one-launch
+# form).
+DECODE_RULE_CASES = [(32, 8, 64, 16, 256), (32, 8, 64, 16, 257), (32, 8, 64, 17, 200), (32, 8, 128, 8, 100), (32, 8, 64, 8, 500), (32, 8, 128, 8, 200), (32, 8, 128, 8, 1000),
                      (24, 8, 128, 3, 350), (32, 32, 128, 1, 1000), (8, 2, 256, 1, 447), (8, 2, 256, 1, 448),
                      (24, 8, 128, 1, 1100)]
 
