@@ -125,6 +125,7 @@ struct RowsCfg {
     static constexpr int kPieces = 4 * kSub;                             // 16-byte pieces per buffered row
     static constexpr int kDma = static_cast<int>(kBuf) / 1024;           // DMA instructions per buffer
     static constexpr int kBatch = kXLds / (kRWaves * 1024);              // accumulator tiles summed per round
+    static_assert((kPieces == 16 || kPieces == 8) && kUnits <= 2, "the swizzle, and the waits of a chunk");
 };
 
 // y_is_f32: 1 stores the f32 sums, 0 their RNE to bf16.
@@ -151,9 +152,7 @@ __global__ __launch_bounds__(kRThreads, 2) void q4_gemm_rows_kernel(
     char *const sbl = rows_smem + C::kXLds + wave * kRSbBytes;
     // slot of piece p in buffered row r: 16 rows of one fragment read hit
     // all 64 banks once
-    auto slot_of = [](uint32_t r, uint32_t p) {
-        return kPieces == 16 ? p ^ (r & 15) : kPieces == 8 ? p ^ ((r >> 1) & 7) : p ^ ((r >> 2) & 3);
-    };
+    auto slot_of = [](uint32_t r, uint32_t p) { return kPieces == 16 ? p ^ (r & 15) : p ^ ((r >> 1) & 7); };
     // DMA instruction d brings 64 / kPieces rows: lane i -> row, slot
     uint32_t xoff[kDma];
 #pragma unroll
@@ -236,10 +235,7 @@ __global__ __launch_bounds__(kRThreads, 2) void q4_gemm_rows_kernel(
             __builtin_amdgcn_sched_barrier(0);
             // this buffer's X has landed: only the requests just made (and,
             // in a chunk's second unit, the next weights) are younger
-            if (u < 2)
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDma + CT) : "memory");
-            else
-                asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDma) : "memory");
+            asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kDma + CT) : "memory");
             __builtin_amdgcn_sched_barrier(0);
             if (u == 0) {
 #pragma unroll
