@@ -172,11 +172,14 @@ static hipError_t trim_pool(fh_device *dev, size_t count) {
 // graph uses. Up to kPoolBlockBytes it is kept for a later fh_alloc (oldest
 // kept blocks make room), else freed. Unless `ordered` says that only ops on
 // the device's stream have touched it, the caller may still be using it on a
-// stream of its own: take_pooled then waits before it goes out again. Every op
-// returns fresh storage, so a program that runs op
-// by op allocates and frees once per op: through the driver that was two
-// host-device round trips an op (14 ops of attention over 512 tokens: 2.5 ms a
-// pass for 0.15 ms of kernels); from kept blocks a pass takes 0.28 ms.
+// stream of its own. That is waited for before it goes out again
+// (take_pooled), or here for a large block while the device's stream is idle:
+// a wait for every stream takes 40 us even then, which a large block's owner
+// has and its next owner, who may have work queued, would pay more for. Every
+// op returns fresh storage, so a program that runs op by op allocates and frees
+// once per op: through the driver that was two host-device round trips an op
+// (14 ops of attention over 512 tokens: 2.5 ms a pass for 0.15 ms of kernels);
+// from kept blocks a pass takes 0.28 ms.
 static hipError_t release(fh_device *dev, uintptr_t base, size_t size, bool ordered) {
     dev->live_bytes -= size;
     const size_t cap = dev->capacity[base];
@@ -191,17 +194,28 @@ static hipError_t release(fh_device *dev, uintptr_t base, size_t size, bool orde
     while (drop < dev->pool.size() && (left > kPoolBytes || dev->pool.size() - drop >= kPoolBlocks))
         left -= dev->pool[drop++].capacity;
     hipError_t err = trim_pool(dev, drop);
-    dev->pool.push_back({base, cap, !ordered});
+    bool shared = !ordered;
+    if (shared && cap >= kSharedWait) {
+        hipError_t werr = hipStreamQuery(dev->stream);
+        if (werr == hipErrorNotReady) {
+            (void)hipGetLastError();
+        } else {
+            if (werr == hipSuccess) werr = hipDeviceSynchronize();
+            if (err == hipSuccess) err = werr;
+            shared = werr != hipSuccess;
+        }
+    }
+    dev->pool.push_back({base, cap, shared});
     dev->pool_bytes += cap;
     return err;
 }
 
 // *out: the smallest kept block that serves `size`, or null. Blocks that may
-// be in use on a caller's stream are left alone while the device's own stream
-// has work, until kSharedBlocks or kSharedBytes of them have gathered; then, as
-// hipFree does, the work queued on every stream of the GPU is waited for, once
-// for all of them. (14 ops of attention over 512 tokens, whose result the caller
-// reads: 276 us a pass, 304 with a wait at each such free.)
+// be in use on a caller's stream are left alone until kSharedBlocks or
+// kSharedBytes of them have gathered; then, as hipFree does, the work queued on
+// every stream of the GPU is waited for, once for all of them. (14 ops of
+// attention over 512 tokens, whose result the caller reads: 276 us a pass, 304
+// with a wait at each such free.)
 static hipError_t take_pooled(fh_device *dev, size_t size, void **out) {
     *out = nullptr;
     const size_t none = dev->pool.size(), most = size + std::max<size_t>(size / 8, kPoolSlack);
@@ -220,12 +234,7 @@ static hipError_t take_pooled(fh_device *dev, size_t size, void **out) {
         }
     }
     if (best == none) {
-        if (!shared_fits) return hipSuccess;
-        if (shared_blocks < kSharedBlocks && shared_bytes < kSharedBytes &&
-            hipStreamQuery(dev->stream) == hipErrorNotReady) {
-            (void)hipGetLastError();
-            return hipSuccess;
-        }
+        if (!shared_fits || (shared_blocks < kSharedBlocks && shared_bytes < kSharedBytes)) return hipSuccess;
         if (hipError_t err = hipDeviceSynchronize(); err != hipSuccess) return err;
         for (PoolBlock &b : dev->pool) b.shared = false;
         return take_pooled(dev, size, out);

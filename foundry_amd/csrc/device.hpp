@@ -55,6 +55,9 @@ constexpr size_t kPoolBlocks = 256;
 // they are waited for (take_pooled).
 constexpr size_t kSharedBlocks = 16;
 constexpr uint64_t kSharedBytes = 16ull << 20;
+// ... and the size from which one is waited for when it is freed, if the
+// device's stream is idle (release).
+constexpr uint64_t kSharedWait = 4ull << 20;
 // A kept block serves a request it exceeds by at most this or 1/8 of it.
 constexpr uint64_t kPoolSlack = 64ull << 10;
 
