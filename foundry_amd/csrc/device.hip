@@ -168,18 +168,44 @@ static hipError_t trim_pool(fh_device *dev, size_t count) {
     return first;
 }
 
+// Every stream of the GPU is waited for: no kept block is in use on one.
+static hipError_t wait_shared(fh_device *dev) {
+    const hipError_t err = hipDeviceSynchronize();
+    if (err == hipSuccess)
+        for (PoolBlock &b : dev->pool) b.shared = false;
+    return err;
+}
+
+// After a block that a caller's stream may use was kept. Frees with no op
+// between them, as when a model or a call's buffers are dropped, mostly find the
+// device's stream idle; the wait for every stream then takes under 1 us, where
+// the next owners would wait for work of their own or allocate anew (the inputs
+// of a 16384 x 3072 linear: 200 us, 360 without this). One that finds the stream
+// busy is left alone, and so is the free of one result between ops: asking costs
+// 25 us after an op.
+static hipError_t settle_shared(fh_device *dev) {
+    const uint64_t now = dev->counters.dispatches;
+    const bool asked = dev->shared_busy_at == now, run = dev->shared_free_at == now;
+    dev->shared_free_at = now;
+    if (!run || asked) return hipSuccess;
+    const hipError_t err = hipStreamQuery(dev->stream);
+    if (err == hipSuccess) return wait_shared(dev);
+    if (err != hipErrorNotReady) return err;
+    (void)hipGetLastError();
+    dev->shared_busy_at = now;
+    return hipSuccess;
+}
+
 // Releases an allocation that is no longer in dev->allocs and that no live
 // graph uses. Up to kPoolBlockBytes it is kept for a later fh_alloc (oldest
 // kept blocks make room), else freed. Unless `ordered` says that only ops on
 // the device's stream have touched it, the caller may still be using it on a
-// stream of its own. That is waited for before it goes out again
-// (take_pooled), or here for a large block while the device's stream is idle:
-// a wait for every stream takes 40 us even then, which a large block's owner
-// has and its next owner, who may have work queued, would pay more for. Every
-// op returns fresh storage, so a program that runs op by op allocates and frees
-// once per op: through the driver that was two host-device round trips an op
-// (14 ops of attention over 512 tokens: 2.5 ms a pass for 0.15 ms of kernels);
-// from kept blocks a pass takes 0.28 ms.
+// stream of its own: that is waited for before it goes out again
+// (take_pooled), or here (settle_shared). Every op returns fresh storage, so a
+// program that runs op by op allocates and frees once per op: through the
+// driver that was two host-device round trips an op (14 ops of attention over
+// 512 tokens: 2.5 ms a pass for 0.15 ms of kernels); from kept blocks a pass
+// takes 0.28 ms.
 static hipError_t release(fh_device *dev, uintptr_t base, size_t size, bool ordered) {
     dev->live_bytes -= size;
     const size_t cap = dev->capacity[base];
@@ -194,19 +220,12 @@ static hipError_t release(fh_device *dev, uintptr_t base, size_t size, bool orde
     while (drop < dev->pool.size() && (left > kPoolBytes || dev->pool.size() - drop >= kPoolBlocks))
         left -= dev->pool[drop++].capacity;
     hipError_t err = trim_pool(dev, drop);
-    bool shared = !ordered;
-    if (shared && cap >= kSharedWait) {
-        hipError_t werr = hipStreamQuery(dev->stream);
-        if (werr == hipErrorNotReady) {
-            (void)hipGetLastError();
-        } else {
-            if (werr == hipSuccess) werr = hipDeviceSynchronize();
-            if (err == hipSuccess) err = werr;
-            shared = werr != hipSuccess;
-        }
-    }
-    dev->pool.push_back({base, cap, shared});
+    dev->pool.push_back({base, cap, !ordered});
     dev->pool_bytes += cap;
+    if (!ordered) {
+        const hipError_t serr = settle_shared(dev);
+        if (err == hipSuccess) err = serr;
+    }
     return err;
 }
 
@@ -235,8 +254,7 @@ static hipError_t take_pooled(fh_device *dev, size_t size, void **out) {
     }
     if (best == none) {
         if (!shared_fits || (shared_blocks < kSharedBlocks && shared_bytes < kSharedBytes)) return hipSuccess;
-        if (hipError_t err = hipDeviceSynchronize(); err != hipSuccess) return err;
-        for (PoolBlock &b : dev->pool) b.shared = false;
+        if (hipError_t err = wait_shared(dev); err != hipSuccess) return err;
         return take_pooled(dev, size, out);
     }
     *out = reinterpret_cast<void *>(dev->pool[best].base);

@@ -55,9 +55,6 @@ constexpr size_t kPoolBlocks = 256;
 // they are waited for (take_pooled).
 constexpr size_t kSharedBlocks = 16;
 constexpr uint64_t kSharedBytes = 16ull << 20;
-// ... and the size from which one is waited for when it is freed, if the
-// device's stream is idle (release).
-constexpr uint64_t kSharedWait = 4ull << 20;
 // A kept block serves a request it exceeds by at most this or 1/8 of it.
 constexpr uint64_t kPoolSlack = 64ull << 10;
 
@@ -84,6 +81,9 @@ struct fh_device {
     // kept (a reused block may exceed the size asked for).
     std::vector<fh::PoolBlock> pool;
     uint64_t pool_bytes = 0;
+    // counters.dispatches at the last free of a shared block, and at the last
+    // that found the stream busy (settle_shared)
+    uint64_t shared_free_at = ~0ull, shared_busy_at = ~0ull;
     std::unordered_map<uintptr_t, size_t> capacity;
     uint64_t live_bytes = 0;
     uint64_t peak_bytes = 0;
