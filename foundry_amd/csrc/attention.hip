@@ -769,7 +769,9 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_chunk_kernel(
 // for attn_combine_kernel. Rows with no key in the chunk write nothing.
 // An inf or NaN of V whose key not every row of the tile attends is staged as
 // 0, since its probability of 0 would make the other rows' sums NaN, and added
-// at the end for the rows that do attend it.
+// at the end for the rows that do attend it. (Looked for as a maximum over the
+// step's exponents, cleared in LDS only where there is one: 512 rows, 24 heads,
+// both kernels 36.1 us without, 36.8 so, 37.5 clearing as the pieces are stored.)
 constexpr int kPvtPitch = 40;  // bf16 per transposed V row in LDS: 32 keys + 8 of padding
 
 template <int HD, int G>
@@ -864,7 +866,19 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
             load_v(s + kAttnWaves, vn);
             load_s(s + kAttnWaves, sn);
         }
-        const bool partly = k0 + s * 32 + 32 > cmin;  // some row does not attend all of the step's keys
+        bool dirty = false;  // an inf or NaN in a step that some row does not attend whole
+        if (k0 + s * 32 + 32 > cmin) {
+            typedef __attribute__((ext_vector_type(2))) uint16_t u16x2_t;
+            u16x2_t most = {0, 0};
+#pragma unroll
+            for (int t = 0; t < 8; ++t) {
+                const uint32_t w[4] = {va[t].x, va[t].y, va[t].z, va[t].w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2_t, w[i] & 0x7FFF7FFFu));
+            }
+            dirty = __any(most.x >= 0x7F80 || most.y >= 0x7F80) != 0;
+        }
         // transpose: dim 8 pv + d of keys 8 vj .. 8 vj + 7 as one 16-byte row piece
 #pragma unroll
         for (int d = 0; d < 8; ++d) {
@@ -876,9 +890,16 @@ __global__ __launch_bounds__(kAttnThreads) void attn_pv_tile_kernel(
                 const uint32_t bw = d / 2 == 0 ? b.x : d / 2 == 1 ? b.y : d / 2 == 2 ? b.z : b.w;
                 w[i] = d % 2 ? (aw >> 16) | (bw & 0xFFFF0000u) : (aw & 0xFFFFu) | (bw << 16);
             }
-            uint4 piece = make_uint4(w[0], w[1], w[2], w[3]);
-            if (partly) cleared |= __any(clear_specials(piece)) != 0;
-            *reinterpret_cast<uint4 *>(&vw[8 * pv + d][8 * vj]) = piece;
+            *reinterpret_cast<uint4 *>(&vw[8 * pv + d][8 * vj]) = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+        if (dirty) {
+            cleared = true;
+#pragma unroll 1
+            for (int d = 0; d < 8; ++d) {
+                uint4 piece = *reinterpret_cast<const uint4 *>(&vw[8 * pv + d][8 * vj]);
+                clear_specials(piece);
+                *reinterpret_cast<uint4 *>(&vw[8 * pv + d][8 * vj]) = piece;
+            }
         }
         // A: the probabilities of keys 8 quad .. 8 quad + 7 of the step for this lane's row
         const uint32_t kb = k0 + s * 32 + 8 * quad;
